@@ -8,6 +8,7 @@
 // point as its temporary grid would hold it) and writes psi_f + dt * rhs_f.
 // Periodic neighbours are found by wrapping coordinates.
 #include "multi.hpp"
+#include "ref_stream.hpp"
 #include "stencil_ref.hpp"
 
 namespace sps {
@@ -165,10 +166,172 @@ __global__ __launch_bounds__(256) void ref_multi_kernel(MRefParams<T> p) {
   }
 }
 
+// ---------------------------------------------------- the step as a row stream
+// (ref_stream.hpp).  Two fields x, y; a right-hand side is a list of
+// coeff * D[x^a y^b] known at compile time, as the models of the reference's
+// MODEL definitions are (examples/models/modeldefinitions.h:74-80,123-136);
+// any other list runs ref_multi_kernel.
+struct MTermForm {
+  int op, a, b;
+};
+struct MForm {
+  int n[2];
+  MTermForm t[2][5];
+};
+constexpr MForm kModelCForm = {
+    {4, 4},
+    {{{SPS_OP_BILAP, 1, 0}, {SPS_OP_LAP, 1, 0}, {SPS_OP_LAP, 3, 0}, {SPS_OP_LAP, 0, 2}},
+     {{SPS_OP_LAP, 0, 1}, {SPS_OP_ID, 0, 1}, {SPS_OP_ID, 0, 3}, {SPS_OP_ID, 1, 1}}}};
+constexpr MForm kGrayScottForm = {
+    {4, 3},
+    {{{SPS_OP_LAP, 1, 0}, {SPS_OP_ID, 1, 2}, {SPS_OP_ID, 0, 0}, {SPS_OP_ID, 1, 0}},
+     {{SPS_OP_LAP, 0, 1}, {SPS_OP_ID, 1, 2}, {SPS_OP_ID, 0, 1}}}};
+constexpr MForm kTuringForm = {
+    {5, 5},
+    {{{SPS_OP_LAP, 1, 0}, {SPS_OP_ID, 1, 0}, {SPS_OP_ID, 0, 1}, {SPS_OP_ID, 1, 2},
+      {SPS_OP_ID, 1, 1}},
+     {{SPS_OP_LAP, 0, 1}, {SPS_OP_ID, 0, 1}, {SPS_OP_ID, 1, 0}, {SPS_OP_ID, 1, 2},
+      {SPS_OP_ID, 1, 1}}}};
+
+constexpr bool form_has(const MForm& f, int op) {
+  for (int e = 0; e < 2; ++e)
+    for (int t = 0; t < f.n[e]; ++t)
+      if (f.t[e][t].op == op) return true;
+  return false;
+}
+
+// x^a y^b as the left fold of its factors in field order, 1 if none
+template <int A, int B, typename T>
+__device__ __forceinline__ T mono(const T (&x)[2]) {
+  if constexpr (A + B == 0) {
+    return T(1);
+  } else {
+    T acc = A > 0 ? x[0] : x[1];
+#pragma unroll
+    for (int j = 1; j < A; ++j) acc = acc * x[0];
+#pragma unroll
+    for (int j = A > 0 ? 0 : 1; j < B; ++j) acc = acc * x[1];
+    return acc;
+  }
+}
+
+template <typename T, const MForm& FORM, int L, int B>
+struct FormStep {
+  static constexpr int NF = 2;
+  // operands under a laplacian that are not a field, in order of appearance
+  struct LapOps {
+    int n = 0;
+    int a[10] = {}, b[10] = {};
+    constexpr LapOps() {
+      for (int e = 0; e < 2; ++e)
+        for (int t = 0; t < FORM.n[e]; ++t)
+          if (FORM.t[e][t].op == SPS_OP_LAP && FORM.t[e][t].a + FORM.t[e][t].b != 1 &&
+              find(FORM.t[e][t].a, FORM.t[e][t].b) < 0) {
+            a[n] = FORM.t[e][t].a;
+            b[n++] = FORM.t[e][t].b;
+          }
+    }
+    constexpr int find(int pa, int pb) const {
+      for (int d = 0; d < n; ++d)
+        if (a[d] == pa && b[d] == pb) return d;
+      return -1;
+    }
+  };
+  static constexpr LapOps kOps{};
+  static constexpr int NLAP = kOps.n;
+  T coeff[2][5];
+  T divh2, divh4, dt;
+
+  template <int d>
+  __device__ __forceinline__ T lap_operand(const T (&x)[2]) const {
+    return mono<kOps.a[d], kOps.b[d]>(x);
+  }
+  template <int S>
+  __device__ __forceinline__ void rhs(
+      const RsWindow<T> (&F)[2], const RsWindow<T> (&D)[NLAP > 0 ? NLAP : 1],
+      const T (&x)[2], T (&r)[2]) const {
+    static_for<0, 2>([&](auto ec) {
+      constexpr int e = decltype(ec)::value;
+      T acc = T(0);
+      static_for<0, FORM.n[e]>([&](auto tc) {
+        constexpr int t = decltype(tc)::value;
+        constexpr MTermForm m = FORM.t[e][t];
+        T v;
+        if constexpr (m.op == SPS_OP_ID) {
+          v = mono<m.a, m.b>(x);
+        } else if constexpr (m.op == SPS_OP_BILAP) {
+          static_assert(m.a + m.b == 1, "the bilaplacian of a field");
+          v = rs_bilap2<T, B>(RsAcc<T, S>{F[m.b]}, divh4);
+        } else if constexpr (m.a + m.b == 1) {
+          v = rs_lap2<T, L>(RsAcc<T, S>{F[m.b]}, divh2);
+        } else {
+          v = rs_lap2<T, L>(RsAcc<T, S>{D[kOps.find(m.a, m.b)]}, divh2);
+        }
+        acc = t == 0 ? coeff[e][t] * v : acc + coeff[e][t] * v;
+      });
+      r[e] = acc;
+    });
+  }
+};
+
+template <typename T>
+bool is_form(const MRefParams<T>& p, const MForm& f) {
+  if (p.nfields != 2) return false;
+  for (int e = 0; e < 2; ++e) {
+    if (p.nterms[e] != f.n[e]) return false;
+    for (int t = 0; t < f.n[e]; ++t)
+      if (p.terms[e][t].op != f.t[e][t].op || p.terms[e][t].pow[0] != f.t[e][t].a ||
+          p.terms[e][t].pow[1] != f.t[e][t].b)
+        return false;
+  }
+  return true;
+}
+
+template <typename T, const MForm& FORM, int L, int B>
+void launch_form_lb(const MRefParams<T>& p, hipStream_t s) {
+  FormStep<T, FORM, L, B> step;
+  RsFields<T, 2> g;
+  for (int e = 0; e < 2; ++e) {
+    for (int t = 0; t < 5; ++t)
+      step.coeff[e][t] = t < FORM.n[e] ? p.terms[e][t].coeff : T(0);
+    g.in[e] = p.in[e];
+    g.out[e] = p.out[e];
+  }
+  step.divh2 = p.divh2;
+  step.divh4 = p.divh4;
+  step.dt = p.dt;
+  g.X = p.n[0];
+  g.Y = p.n[1];
+  launch_ref_stream2d(g, step, s);
+}
+
+template <typename T, const MForm& FORM, int L>
+void launch_form_l(const MRefParams<T>& p, hipStream_t s) {
+  if constexpr (!form_has(FORM, SPS_OP_BILAP)) {
+    launch_form_lb<T, FORM, L, 13>(p, s);
+  } else {
+    if (p.B == 13) launch_form_lb<T, FORM, L, 13>(p, s);
+    else if (p.B == 17) launch_form_lb<T, FORM, L, 17>(p, s);
+    else launch_form_lb<T, FORM, L, 21>(p, s);
+  }
+}
+
+template <typename T, const MForm& FORM>
+bool launch_form(const MRefParams<T>& p, hipStream_t s) {
+  if (!is_form(p, FORM)) return false;
+  if (p.L == 5) launch_form_l<T, FORM, 5>(p, s);
+  else launch_form_l<T, FORM, 9>(p, s);
+  return true;
+}
+
 }  // namespace
 
 template <typename T>
 int launch_ref_multi(const MRefParams<T>& p, int dim, hipStream_t stream) {
+  if (dim == 2 && (launch_form<T, kModelCForm>(p, stream) ||
+                   launch_form<T, kGrayScottForm>(p, stream) ||
+                   launch_form<T, kTuringForm>(p, stream)))
+    return SPS_OK;
   dim3 block(64, 4, 1);
   dim3 grid((p.n[0] + 63) / 64, (p.n[1] + 3) / 4, dim == 3 ? p.n[2] : 1);
   if (dim == 2)
