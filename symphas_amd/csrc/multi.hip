@@ -99,7 +99,19 @@ __device__ __forceinline__ void eval_poly(int cls,
 // first stage keeps the unscaled D(psi_f) and its update is
 // psi_f + Adt_f + k1_f * D(psi_f), k1_f = kd * b_f: the radius-one form, run
 // in step with the other field's two stages.
-template <typename T, int VEC, int R, int LIN>
+// Classes the polynomials of a kernel instance have (kPoly..., or kPolyAny:
+// the class is the kernel argument's).  With the classes known the stages are
+// one straight block; with kPolyAny every evaluation carries the code of all
+// seven classes and a branch to the right one, which keeps the scheduler from
+// overlapping the two fields and, at four steps, fills the instruction cache.
+constexpr int kPolyAny = -1;
+template <int A0, int A1, int B0, int B1>
+struct PolyClasses {
+  static constexpr int a[2] = {A0, A1}, b[2] = {B0, B1};
+};
+using AnyClasses = PolyClasses<kPolyAny, kPolyAny, kPolyAny, kPolyAny>;
+
+template <typename T, int VEC, int R, int LIN, class PC>
 struct Stage2 {
   T P[2][3][VEC];  // input rows of both fields (slots rotate with the phase)
   T M[2][3][VEC];  // mu rows (radius 2)
@@ -126,6 +138,14 @@ struct Stage2 {
     }
   }
 
+  // polynomial f of a set (c, with its classes) at rows x, y
+  template <int CLS>
+  __device__ __forceinline__ static void poly(
+      int cls, const T (&c)[kMDeg + 1][kMDeg + 1], const T* x, const T* y,
+      T* p) {
+    eval_poly<T, VEC>(CLS == kPolyAny ? cls : CLS, c, x, y, p);
+  }
+
   template <int PH>
   __device__ __forceinline__ void push(const MFusedCoef<T>& c,
                                        T (&v)[2][VEC]) {
@@ -138,8 +158,8 @@ struct Stage2 {
     diff5<S1, S2, S0>(P[0], d[0]);
     diff5<S1, S2, S0>(P[1], d[1]);
     if constexpr (R == 1) {
-      eval_poly<T, VEC>(c.adt_class[0], c.adt[0], P[0][S1], P[1][S1], a[0]);
-      eval_poly<T, VEC>(c.adt_class[1], c.adt[1], P[0][S1], P[1][S1], a[1]);
+      poly<PC::a[0]>(c.adt_class[0], c.adt[0], P[0][S1], P[1][S1], a[0]);
+      poly<PC::a[1]>(c.adt_class[1], c.adt[1], P[0][S1], P[1][S1], a[1]);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
         v[0][j] = fmad(c.k1[0], d[0][j], P[0][S1][j] + a[0][j]);
@@ -148,9 +168,9 @@ struct Stage2 {
     } else {
       constexpr bool lin0 = LIN == 2, lin1 = LIN == 1;
       if constexpr (!lin0)
-        eval_poly<T, VEC>(c.b_class[0], c.b[0], P[0][S1], P[1][S1], a[0]);
+        poly<PC::b[0]>(c.b_class[0], c.b[0], P[0][S1], P[1][S1], a[0]);
       if constexpr (!lin1)
-        eval_poly<T, VEC>(c.b_class[1], c.b[1], P[0][S1], P[1][S1], a[1]);
+        poly<PC::b[1]>(c.b_class[1], c.b[1], P[0][S1], P[1][S1], a[1]);
 #pragma unroll
       for (int f = 0; f < 2; ++f) {
         const bool lin = f == 0 ? lin0 : lin1;
@@ -160,8 +180,8 @@ struct Stage2 {
       }
       if constexpr (!lin0) diff5<S1, S2, S0>(M[0], d[0]);
       if constexpr (!lin1) diff5<S1, S2, S0>(M[1], d[1]);
-      eval_poly<T, VEC>(c.adt_class[0], c.adt[0], P[0][S0], P[1][S0], a[0]);
-      eval_poly<T, VEC>(c.adt_class[1], c.adt[1], P[0][S0], P[1][S0], a[1]);
+      poly<PC::a[0]>(c.adt_class[0], c.adt[0], P[0][S0], P[1][S0], a[0]);
+      poly<PC::a[1]>(c.adt_class[1], c.adt[1], P[0][S0], P[1][S0], a[1]);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
         v[0][j] = lin0 ? fmad(c.k1[0], M[0][S1][j], P[0][S0][j] + a[0][j])
@@ -173,17 +193,17 @@ struct Stage2 {
   }
 };
 
-template <typename T, int VEC, int K, int R, int LIN>
-__global__ __launch_bounds__(256) void fused_multi(
+template <typename T, int VEC, int K, int R, int LIN, class PC>
+__global__ __launch_bounds__(64) void fused_multi(
     const T* __restrict__ in0, const T* __restrict__ in1, T* __restrict__ out0,
     T* __restrict__ out1, int X, int Y, int TY, int nstrips, int nitems,
     MFusedCoef<T> c) {
   constexpr int HL = (K * R + VEC - 1) / VEC;
   constexpr int W = (64 - 2 * HL) * VEC;
   constexpr int LAG = K * R;
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x;
   const int item = __builtin_amdgcn_readfirstlane(
-      xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6));
+      xcd_remap(blockIdx.x, gridDim.x));
   if (item >= nitems) return;
   const int strip = item % nstrips;
   const int chunk = item / nstrips;
@@ -197,7 +217,7 @@ __global__ __launch_bounds__(256) void fused_multi(
   int rload = (y0 - LAG) % Y;
   if (rload < 0) rload += Y;
 
-  Stage2<T, VEC, R, LIN> st[K];
+  Stage2<T, VEC, R, LIN, PC> st[K];
 #pragma unroll
   for (int s = 0; s < K; ++s) st[s].clear();
 
@@ -268,7 +288,7 @@ __global__ __launch_bounds__(256) void fused_multi(
   }
 }
 
-template <typename T, int VEC, int K, int R, int LIN>
+template <typename T, int VEC, int K, int R, int LIN, class PC>
 int launch_multi_v(const T* const* in, T* const* out, int X, int Y, int TY,
                    const MFusedCoef<T>& c, hipStream_t s) {
   constexpr int HL = (K * R + VEC - 1) / VEC;
@@ -276,54 +296,71 @@ int launch_multi_v(const T* const* in, T* const* out, int X, int Y, int TY,
   const int nstrips = (X + W - 1) / W;
   const int nchunks = (Y + TY - 1) / TY;
   const int nitems = nstrips * nchunks;
-  fused_multi<T, VEC, K, R, LIN><<<(nitems + 3) / 4, 256, 0, s>>>(
+  fused_multi<T, VEC, K, R, LIN, PC><<<nitems, 64, 0, s>>>(
       in[0], in[1], out[0], out[1], X, Y, TY, nstrips, nitems, c);
   return SPS_OK;
 }
 
-// 16-byte lanes (VEC = 16 / sizeof(T)) or 8-byte lanes (VEC = 8 / sizeof(T))
-template <typename T, int K, int R, int LIN>
-int launch_multi_k(const T* const* in, T* const* out, int X, int Y, int TY,
-                   int vec, const MFusedCoef<T>& c, hipStream_t s) {
-  if (vec == 16 / (int)sizeof(T))
-    return launch_multi_v<T, 16 / sizeof(T), K, R, LIN>(in, out, X, Y, TY, c, s);
-  return launch_multi_v<T, 8 / sizeof(T), K, R, LIN>(in, out, X, Y, TY, c, s);
+// Picks the kernel instance of (radius, linear field, polynomial classes) for
+// c and calls f.template run<R, LIN, PC>().  The instances with known classes
+// are those of the reference's coupled models: both pointwise polynomials
+// linear in the first field (Gray-Scott, Turing), and Model C, whose conserved
+// field's B is separable and whose other field is linear and has a pointwise
+// polynomial linear in the conserved one (either field order).
+// Known classes against kPolyAny, 4096^2 FP32 at the best shape of each:
+// Gray-Scott (4 steps) 17.9 -> 12.9 us per step, Model C (2 steps) 26.1 ->
+// 23.5; 64^2: 2.49 -> 1.34 and 3.92 -> 2.80.
+template <typename T, class F>
+auto with_classes(const MFusedCoef<T>& c, const F& f) {
+  using XX = PolyClasses<kPolyXLin, kPolyXLin, kPolyAny, kPolyAny>;
+  using C1 = PolyClasses<kPolyZero, kPolyXLin, kPolySep, kPolyAny>;
+  using C2 = PolyClasses<kPolyYLin, kPolyZero, kPolyAny, kPolySep>;
+  const int a0 = c.adt_class[0], a1 = c.adt_class[1];
+  if (c.radius == 1)
+    return a0 == kPolyXLin && a1 == kPolyXLin ? f.template run<1, 0, XX>()
+                                              : f.template run<1, 0, AnyClasses>();
+  if (c.lin == 1)
+    return a0 == kPolyZero && a1 == kPolyXLin && c.b_class[0] == kPolySep
+               ? f.template run<2, 1, C1>()
+               : f.template run<2, 1, AnyClasses>();
+  if (c.lin == 2)
+    return a0 == kPolyYLin && a1 == kPolyZero && c.b_class[1] == kPolySep
+               ? f.template run<2, 2, C2>()
+               : f.template run<2, 2, AnyClasses>();
+  return f.template run<2, 0, AnyClasses>();
 }
 
 template <typename T, int K>
-int launch_multi_r(const T* const* in, T* const* out, int X, int Y, int TY,
-                   int vec, const MFusedCoef<T>& c, hipStream_t s) {
-  if (c.radius == 1) return launch_multi_k<T, K, 1, 0>(in, out, X, Y, TY, vec, c, s);
-  if (c.lin == 1) return launch_multi_k<T, K, 2, 1>(in, out, X, Y, TY, vec, c, s);
-  if (c.lin == 2) return launch_multi_k<T, K, 2, 2>(in, out, X, Y, TY, vec, c, s);
-  return launch_multi_k<T, K, 2, 0>(in, out, X, Y, TY, vec, c, s);
-}
+struct MultiLaunch {
+  const T* const* in;
+  T* const* out;
+  int X, Y, TY, vec;
+  const MFusedCoef<T>& c;
+  hipStream_t s;
+  template <int R, int LIN, class PC>
+  int run() const {
+    return vec == 16 / (int)sizeof(T)
+               ? launch_multi_v<T, 16 / sizeof(T), K, R, LIN, PC>(in, out, X, Y, TY, c, s)
+               : launch_multi_v<T, 8 / sizeof(T), K, R, LIN, PC>(in, out, X, Y, TY, c, s);
+  }
+};
 
 // Private-segment (scratch) bytes per lane of one kernel instance, as the
 // compiler's resource report records it: nonzero when the instance spills
 // its registers to scratch memory.
-template <typename T, int VEC, int K, int R, int LIN>
-size_t multi_scratch_v() {
-  hipFuncAttributes a{};
-  if (hipFuncGetAttributes(&a, (const void*)fused_multi<T, VEC, K, R, LIN>) !=
-      hipSuccess)
-    return 0;
-  return a.localSizeBytes;
-}
-
-template <typename T, int K, int R, int LIN>
-size_t multi_scratch_k(int vec) {
-  if (vec == 16 / (int)sizeof(T)) return multi_scratch_v<T, 16 / sizeof(T), K, R, LIN>();
-  return multi_scratch_v<T, 8 / sizeof(T), K, R, LIN>();
-}
-
 template <typename T, int K>
-size_t multi_scratch_r(int vec, const MFusedCoef<T>& c) {
-  if (c.radius == 1) return multi_scratch_k<T, K, 1, 0>(vec);
-  if (c.lin == 1) return multi_scratch_k<T, K, 2, 1>(vec);
-  if (c.lin == 2) return multi_scratch_k<T, K, 2, 2>(vec);
-  return multi_scratch_k<T, K, 2, 0>(vec);
-}
+struct MultiScratch {
+  int vec;
+  template <int R, int LIN, class PC>
+  size_t run() const {
+    const void* k =
+        vec == 16 / (int)sizeof(T)
+            ? (const void*)fused_multi<T, 16 / sizeof(T), K, R, LIN, PC>
+            : (const void*)fused_multi<T, 8 / sizeof(T), K, R, LIN, PC>;
+    hipFuncAttributes a{};
+    return hipFuncGetAttributes(&a, k) == hipSuccess ? a.localSizeBytes : 0;
+  }
+};
 
 }  // namespace
 
@@ -332,10 +369,10 @@ size_t multi_scratch_r(int vec, const MFusedCoef<T>& c) {
 template <typename T>
 size_t fused_multi_scratch(int K, int vec, const MFusedCoef<T>& c) {
   switch (K) {
-    case 1: return multi_scratch_r<T, 1>(vec, c);
-    case 2: return multi_scratch_r<T, 2>(vec, c);
-    case 3: return multi_scratch_r<T, 3>(vec, c);
-    case 4: return multi_scratch_r<T, 4>(vec, c);
+    case 1: return with_classes(c, MultiScratch<T, 1>{vec});
+    case 2: return with_classes(c, MultiScratch<T, 2>{vec});
+    case 3: return with_classes(c, MultiScratch<T, 3>{vec});
+    case 4: return with_classes(c, MultiScratch<T, 4>{vec});
     default: return 0;
   }
 }
@@ -353,10 +390,10 @@ int launch_fused_multi(const T* const* in, T* const* out, int X, int Y, int K,
   }
   int rc;
   switch (K) {
-    case 1: rc = launch_multi_r<T, 1>(in, out, X, Y, TY, vec, c, s); break;
-    case 2: rc = launch_multi_r<T, 2>(in, out, X, Y, TY, vec, c, s); break;
-    case 3: rc = launch_multi_r<T, 3>(in, out, X, Y, TY, vec, c, s); break;
-    case 4: rc = launch_multi_r<T, 4>(in, out, X, Y, TY, vec, c, s); break;
+    case 1: rc = with_classes(c, MultiLaunch<T, 1>{in, out, X, Y, TY, vec, c, s}); break;
+    case 2: rc = with_classes(c, MultiLaunch<T, 2>{in, out, X, Y, TY, vec, c, s}); break;
+    case 3: rc = with_classes(c, MultiLaunch<T, 3>{in, out, X, Y, TY, vec, c, s}); break;
+    case 4: rc = with_classes(c, MultiLaunch<T, 4>{in, out, X, Y, TY, vec, c, s}); break;
     default:
       set_error("fused coupled step: steps per launch %d not in 1..4", K);
       return SPS_E_INVALID;
@@ -393,6 +430,13 @@ __device__ __forceinline__ T d7m(const T (&a)[3][NI], int r) {
                   (a[S0][r + 1] + a[S2][r + 1]));
 }
 
+template <int CLS, typename T>
+__device__ __forceinline__ void poly3(int cls,
+                                      const T (&c)[kMDeg + 1][kMDeg + 1], T x,
+                                      T y, T& p) {
+  eval_poly<T, 1>(CLS == kPolyAny ? cls : CLS, c, &x, &y, &p);
+}
+
 template <int N>
 struct MRowsOf {
   static constexpr int value = N > 0 ? N : 1;
@@ -402,7 +446,7 @@ struct MRowsOf {
 // owns 64 columns (one per lane, R*K halo lanes per side) x TYW rows of a
 // z-chunk; K steps are a chain of radius-one stages (radius two: mu, then
 // update), every stage carrying both fields in rings of three planes.
-template <typename T, int TYW, int R, int K, int LIN>
+template <typename T, int TYW, int R, int K, int LIN, class PC>
 __global__ __launch_bounds__(256) void fused3d_multi(
     const T* __restrict__ in0, const T* __restrict__ in1, T* __restrict__ out0,
     T* __restrict__ out1, int X, int Y, int Z, int TZ, int nstrips, int nrowblk,
@@ -488,8 +532,8 @@ __global__ __launch_bounds__(256) void fused3d_multi(
       if constexpr (MU) {
         const T xv = a[0][S1][r + 1], yv = a[1][S1][r + 1];
         T p0 = T(0), p1 = T(0);
-        if constexpr (!lin0) eval_poly<T, 1>(c.b_class[0], c.b[0], &xv, &yv, &p0);
-        if constexpr (!lin1) eval_poly<T, 1>(c.b_class[1], c.b[1], &xv, &yv, &p1);
+        if constexpr (!lin0) poly3<PC::b[0]>(c.b_class[0], c.b[0], xv, yv, p0);
+        if constexpr (!lin1) poly3<PC::b[1]>(c.b_class[1], c.b[1], xv, yv, p1);
         res[0][r] = lin0 ? d0 : fmad(c.kmu[0], d0, p0);
         res[1][r] = lin1 ? d1 : fmad(c.kmu[1], d1, p1);
       } else {
@@ -502,8 +546,8 @@ __global__ __launch_bounds__(256) void fused3d_multi(
           yv = a[1][S1][r + 1];
         }
         T p0, p1;
-        eval_poly<T, 1>(c.adt_class[0], c.adt[0], &xv, &yv, &p0);
-        eval_poly<T, 1>(c.adt_class[1], c.adt[1], &xv, &yv, &p1);
+        poly3<PC::a[0]>(c.adt_class[0], c.adt[0], xv, yv, p0);
+        poly3<PC::a[1]>(c.adt_class[1], c.adt[1], xv, yv, p1);
         res[0][r] = lin0 ? fmad(c.k1[0], a[0][S1][r + 1], xv + p0)
                          : fmad(R == 2 ? c.kd : c.k1[0], d0, xv + p0);
         res[1][r] = lin1 ? fmad(c.k1[1], a[1][S1][r + 1], yv + p1)
@@ -557,7 +601,7 @@ __global__ __launch_bounds__(256) void fused3d_multi(
   }
 }
 
-template <typename T, int TYW, int R, int K, int LIN>
+template <typename T, int TYW, int R, int K, int LIN, class PC>
 int launch3m(const T* const* in, T* const* out, int X, int Y, int Z, int TZ,
              const MFusedCoef<T>& c, hipStream_t s) {
   constexpr int W = 64 - 2 * R * K;
@@ -569,11 +613,30 @@ int launch3m(const T* const* in, T* const* out, int X, int Y, int Z, int TZ,
     set_error("fused coupled 3D step: too many work items");
     return SPS_E_INVALID;
   }
-  fused3d_multi<T, TYW, R, K, LIN><<<(unsigned)((nitems + 3) / 4), 256, 0, s>>>(
+  fused3d_multi<T, TYW, R, K, LIN, PC><<<(unsigned)((nitems + 3) / 4), 256, 0, s>>>(
       in[0], in[1], out[0], out[1], X, Y, Z, TZ, nstrips, nrowblk, (int)nitems,
       c);
   return SPS_OK;
 }
+
+
+template <typename T>
+struct Multi3Launch {
+  const T* const* in;
+  T* const* out;
+  int X, Y, Z, K, TY, TZ;
+  const MFusedCoef<T>& c;
+  hipStream_t s;
+  template <int R, int LIN, class PC>
+  int run() const {
+    if constexpr (R == 1)
+      if (K == 2)
+        return TY == 4 ? launch3m<T, 4, R, 2, LIN, PC>(in, out, X, Y, Z, TZ, c, s)
+                       : launch3m<T, 8, R, 2, LIN, PC>(in, out, X, Y, Z, TZ, c, s);
+    return TY == 4 ? launch3m<T, 4, R, 1, LIN, PC>(in, out, X, Y, Z, TZ, c, s)
+                   : launch3m<T, 8, R, 1, LIN, PC>(in, out, X, Y, Z, TZ, c, s);
+  }
+};
 
 }  // namespace
 
@@ -591,24 +654,7 @@ int launch_fused3d_multi(const T* const* in, T* const* out, int X, int Y,
               TY);
     return SPS_E_INVALID;
   }
-  int rc;
-  if (c.radius == 1) {
-    if (K == 1)
-      rc = TY == 4 ? launch3m<T, 4, 1, 1, 0>(in, out, X, Y, Z, TZ, c, s)
-                   : launch3m<T, 8, 1, 1, 0>(in, out, X, Y, Z, TZ, c, s);
-    else
-      rc = TY == 4 ? launch3m<T, 4, 1, 2, 0>(in, out, X, Y, Z, TZ, c, s)
-                   : launch3m<T, 8, 1, 2, 0>(in, out, X, Y, Z, TZ, c, s);
-  } else if (c.lin == 1) {
-    rc = TY == 4 ? launch3m<T, 4, 2, 1, 1>(in, out, X, Y, Z, TZ, c, s)
-                 : launch3m<T, 8, 2, 1, 1>(in, out, X, Y, Z, TZ, c, s);
-  } else if (c.lin == 2) {
-    rc = TY == 4 ? launch3m<T, 4, 2, 1, 2>(in, out, X, Y, Z, TZ, c, s)
-                 : launch3m<T, 8, 2, 1, 2>(in, out, X, Y, Z, TZ, c, s);
-  } else {
-    rc = TY == 4 ? launch3m<T, 4, 2, 1, 0>(in, out, X, Y, Z, TZ, c, s)
-                 : launch3m<T, 8, 2, 1, 0>(in, out, X, Y, Z, TZ, c, s);
-  }
+  const int rc = with_classes(c, Multi3Launch<T>{in, out, X, Y, Z, K, TY, TZ, c, s});
   if (rc != SPS_OK) return rc;
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
