@@ -20,6 +20,7 @@
 #include "energy.hpp"
 #include "fused_tile.hpp"
 #include "plan.hpp"
+#include "reduce_rows.hpp"
 
 namespace sps {
 namespace {
@@ -90,47 +91,47 @@ __global__ __launch_bounds__(256) void batch_kernel(
   }
 }
 
-// FP64 sums per instance: one workgroup per instance, each with the free-
-// energy functional set for it (energy.hpp).
+// FP64 sums per instance, each with the free-energy functional set for it
+// (energy.hpp): kRedParts workgroups per instance take equal ranges of its
+// rows, then one wave adds an instance's parts in order.  With one workgroup
+// per instance the largest of the batch set the time: 256 instances of 128^2
+// to 512^2 took 0.48 ms.
+constexpr int kRedParts = 16;
+
 __global__ __launch_bounds__(256) void batch_reduce(
     const BatchInst* __restrict__ insts, const EnergyParams* __restrict__ eps,
-    int parity, double* __restrict__ out) {
-  const BatchInst& I = insts[blockIdx.x];
-  const EnergyParams ep = eps[blockIdx.x];
-  const float* f = I.buf[parity];
+    int parity, double* __restrict__ part) {
+  const int i = blockIdx.x / kRedParts, c = blockIdx.x % kRedParts;
+  const BatchInst& I = insts[i];
+  const EnergyParams ep = eps[i];
   const int X = I.X, Y = I.Y;
-  const bool central = ep.central != 0;
+  const int r0 = (int)((int64_t)Y * c / kRedParts);
+  const int r1 = (int)((int64_t)Y * (c + 1) / kRedParts);
   double m = 0.0, e = 0.0;
-  for (int y = 0; y < Y; ++y) {
-    const float* row = f + (int64_t)y * X;
-    const float* rowyn = f + (int64_t)(y + 1 == Y ? 0 : y + 1) * X;
-    const float* rowyp =
-        central ? f + (int64_t)(y == 0 ? Y - 1 : y - 1) * X : row;
-    for (int x = threadIdx.x; x < X; x += 256) {
-      const double p = row[x];
-      const int xp = central ? (x == 0 ? X - 1 : x - 1) : x;
-      const double gx = (double)row[x + 1 == X ? 0 : x + 1] - (double)row[xp];
-      const double gy = (double)rowyn[x] - (double)rowyp[x];
-      m += p;
-      e += landau_density(ep, p, gx * gx + gy * gy);
-    }
-  }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) {
-    m += __shfl_xor(m, o, 64);
-    e += __shfl_xor(e, o, 64);
-  }
-  __shared__ double sh[2][4];
-  if ((threadIdx.x & 63) == 0) {
-    sh[0][threadIdx.x >> 6] = m;
-    sh[1][threadIdx.x >> 6] = e;
-  }
-  __syncthreads();
+  if (X % 4 == 0)
+    reduce_rows<float, 4>(I.buf[parity], 2, X, Y, 1, r0, r1, ep, m, e);
+  else
+    reduce_rows<float, 2>(I.buf[parity], 2, X, Y, 1, r0, r1, ep, m, e);
+  block_sum2<4>(m, e);
   if (threadIdx.x == 0) {
-    out[2 * blockIdx.x] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
-    out[2 * blockIdx.x + 1] = ((sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3])) *
-                              (ep.mean ? 1.0 / ((double)X * Y) : I.h * I.h);
+    part[2 * blockIdx.x] = m;
+    part[2 * blockIdx.x + 1] = e;
   }
+}
+
+__global__ __launch_bounds__(64) void batch_reduce_parts(
+    const BatchInst* __restrict__ insts, const EnergyParams* __restrict__ eps,
+    int count, const double* __restrict__ part, double* __restrict__ out) {
+  const int i = blockIdx.x * 64 + threadIdx.x;
+  if (i >= count) return;
+  double m = 0.0, e = 0.0;
+  for (int c = 0; c < kRedParts; ++c) {
+    m += part[2 * (i * kRedParts + c)];
+    e += part[2 * (i * kRedParts + c) + 1];
+  }
+  const BatchInst& I = insts[i];
+  out[2 * i] = m;
+  out[2 * i + 1] = e * (eps[i].mean ? 1.0 / ((double)I.X * I.Y) : I.h * I.h);
 }
 
 int kind_of(const FusedCoef<float>& c) {
@@ -154,7 +155,7 @@ struct sps_fd_batch {
   float* pool = nullptr;  // 2 * total floats
   BatchInst* d_insts = nullptr;
   BatchItem* d_items[4] = {};  // item table per steps-per-launch (strip widths differ)
-  double* d_red = nullptr;
+  double* d_red = nullptr;  // sums per instance, then their parts
   EnergyParams* d_energy = nullptr;  // per-instance free-energy functional
   int nitems[4] = {};
   int parity = 0;
@@ -368,7 +369,8 @@ int sps_fd_batch_create(const sps_fd_desc* descs, int count,
   if (hipMalloc(&b->d_insts, sizeof(BatchInst) * count) != hipSuccess ||
       hipMemcpy(b->d_insts, b->h_insts.data(), sizeof(BatchInst) * count,
                 hipMemcpyHostToDevice) != hipSuccess ||
-      hipMalloc(&b->d_red, 2 * sizeof(double) * count) != hipSuccess ||
+      hipMalloc(&b->d_red, 2 * sizeof(double) * count * (1 + kRedParts)) !=
+          hipSuccess ||
       hipMalloc(&b->d_energy, sizeof(EnergyParams) * count) != hipSuccess) {
     set_error("batch device set-up failed");
     return fail(SPS_E_HIP);
@@ -485,8 +487,11 @@ int sps_fd_batch_reduce(sps_fd_batch* b, double* mass, double* energy) {
     set_error("batch is NULL");
     return SPS_E_INVALID;
   }
-  batch_reduce<<<b->count, 256, 0, b->stream>>>(b->d_insts, b->d_energy,
-                                                 b->parity, b->d_red);
+  double* part = b->d_red + 2 * (size_t)b->count;
+  batch_reduce<<<(unsigned)b->count * kRedParts, 256, 0, b->stream>>>(
+      b->d_insts, b->d_energy, b->parity, part);
+  batch_reduce_parts<<<((unsigned)b->count + 63) / 64, 64, 0, b->stream>>>(
+      b->d_insts, b->d_energy, b->count, part, b->d_red);
   SPS_HIP_TRY(hipGetLastError());
   std::vector<double> h(2 * (size_t)b->count);
   SPS_HIP_TRY(hipMemcpyAsync(h.data(), b->d_red, h.size() * sizeof(double),
