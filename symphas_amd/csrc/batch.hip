@@ -13,6 +13,8 @@
 // replayed.
 #include <algorithm>
 #include <cstring>
+#include <functional>
+#include <map>
 #include <new>
 #include <vector>
 
@@ -21,6 +23,7 @@
 #include "fused_tile.hpp"
 #include "plan.hpp"
 #include "reduce_rows.hpp"
+#include "shape.hpp"
 
 namespace sps {
 namespace {
@@ -68,19 +71,22 @@ __device__ __forceinline__ void run_strip(const BatchInst& I, int parity,
 }
 
 // Persistent: a grid of resident waves walks the item list (strip x row
-// chunk, near-uniform in cost) with a static stride, so no counter or atomic
-// is needed; consecutive blocks go to one XCD.  Every wave's loop bound is
-// nitems, which it reaches.
+// chunk) with a static stride, so no counter or atomic is needed.  Workgroup b
+// runs on XCD b mod 8; the list (build_items) gives every XCD whole instances,
+// or contiguous pieces of them, of like total cost, the costliest items first,
+// so that halo rows stay in one L2 and the CUs' loads stay even.  Every wave's
+// loop bound is nitems, which it reaches.
 template <int K>
 __global__ __launch_bounds__(256) void batch_kernel(
     const BatchInst* __restrict__ insts, const BatchItem* __restrict__ items,
     int nitems, int parity) {
   const int lane = threadIdx.x & 63;
-  const int first = __builtin_amdgcn_readfirstlane(
-      xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6));
+  const int first =
+      __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
   const int stride = (int)gridDim.x * 4;
   for (int it = first; it < nitems; it += stride) {
     const BatchItem item = items[it];
+    if (item.ty == 0) continue;  // filler of an XCD's shorter list
     const BatchInst& I = insts[item.inst];
     switch (I.kind) {
       case 0: run_strip<K, 1, true>(I, parity, item, lane); break;
@@ -159,9 +165,7 @@ struct sps_fd_batch {
   EnergyParams* d_energy = nullptr;  // per-instance free-energy functional
   int nitems[4] = {};
   int parity = 0;
-  // 4 steps x 64-row chunks: best on 256 mixed instances (1.61 T site-updates/s;
-  // 32-row chunks give more items than resident waves and a second round)
-  int K = 4, TY = 64;
+  int K = 4, TY = 64;  // TY: choose_rows
   bool has_data = false;
   GraphSlot graphs[2];
   std::vector<BatchInst> h_insts;
@@ -178,29 +182,118 @@ struct sps_fd_batch {
   long count_items(int k, int ty) const {
     long n = 0;
     for (int i = 0; i < count; ++i) {
-      const int R = (h_insts[i].kind == 1 || h_insts[i].kind == 2) ? 2 : 1;
-      const int W = batch_strip_width(k, R);
+      const int W = batch_strip_width(k, radius_of(i));
       n += (long)((descs[i].n[0] + W - 1) / W) * ((descs[i].n[1] + ty - 1) / ty);
     }
     return n;
   }
 
-  int build_items() {
-    for (int k = 1; k <= 4; ++k) {
-      std::vector<BatchItem> items;
+  int radius_of(int i) const {
+    return (h_insts[i].kind == 1 || h_insts[i].kind == 2) ? 2 : 1;
+  }
+  // cost of streaming a chunk of ty rows, K steps: the rows and the fill, a
+  // radius-two row 10 to a radius-one row's 9
+  static int item_cost(int k, int R, int ty) {
+    return (ty + 2 * k * R) * (R == 2 ? 10 : 9);
+  }
+
+  // Item height before any tuning: between the mean load of a SIMD and the
+  // load of one that gets the first item of every layer of kSimds items, taken
+  // costliest first; a lone item's rows cost 1.5 of a shared one's (their
+  // latency shows).  256 mixed instances, us per 4-step launch at 48 / 64 / 86
+  // / 96 / 128 rows: 48.2 / 48.8 / 45.3 / 46.3 / 49.6 (96 is picked); the list
+  // sorted over the whole chip instead of per XCD 53.9 / 53.1 / 49.3 / 52.1 /
+  // 51.4.
+  void choose_rows() {
+    int64_t least = 0;
+    for (int rows : {4, 6, 8, 12, 16, 24, 32, 43, 48, 64, 86, 96, 103, 128, 171, 256, 512}) {
+      std::map<int, int64_t, std::greater<int>> hist;  // cost -> items
       for (int i = 0; i < count; ++i) {
-        const int R = (h_insts[i].kind == 1 || h_insts[i].kind == 2) ? 2 : 1;
-        const int W = batch_strip_width(k, R);
+        const int R = radius_of(i), W = batch_strip_width(K, R);
         const int X = descs[i].n[0], Y = descs[i].n[1];
-        for (int st = 0; st * W < X; ++st)
-          for (int y0 = 0; y0 < Y; y0 += TY)
-            items.push_back(BatchItem{i, y0, std::min(TY, Y - y0), st});
+        const int64_t strips = (X + W - 1) / W;
+        if (Y / rows) hist[item_cost(K, R, rows)] += strips * (Y / rows);
+        if (Y % rows) hist[item_cost(K, R, Y % rows)] += strips;
       }
-      // largest first: cost ~ streamed rows (every strip is equally wide)
-      std::stable_sort(items.begin(), items.end(),
-                       [](const BatchItem& a, const BatchItem& b) {
-                         return a.ty > b.ty;
-                       });
+      int64_t layers = 0, all = 0, next = 0, seen = 0;
+      for (const auto& h : hist) {
+        seen += h.second;
+        all += h.first * h.second;
+        for (; next < seen; next += kSimds) layers += h.first;
+      }
+      const int64_t cost = std::max((all / kSimds + layers) / 2,
+                                    hist.begin()->first * (int64_t)3 / 2);
+      if (least == 0 || cost < least) {
+        least = cost;
+        TY = rows;
+      }
+    }
+  }
+
+  // The item list of each steps-per-launch, for the batch's item height.
+  int build_items() {
+    constexpr int kXcds = 8, kWaves = 4;  // kWaves: of a workgroup
+    for (int k = 1; k <= 4; ++k) {
+      // units of work that stay together: an instance, or a piece of one that
+      // is more than 1/64 of the batch
+      struct Unit {
+        int64_t cost;
+        std::vector<BatchItem> items;
+      };
+      auto cost = [&](const BatchItem& it) {
+        return (int64_t)item_cost(k, radius_of(it.inst), it.ty);
+      };
+      std::vector<Unit> units;
+      int64_t total = 0;
+      for (int i = 0; i < count; ++i) {
+        const int W = batch_strip_width(k, radius_of(i));
+        const int X = descs[i].n[0], Y = descs[i].n[1];
+        units.push_back(Unit{0, {}});
+        for (int st = 0; st * W < X; ++st)
+          for (int y0 = 0; y0 < Y; y0 += TY) {
+            const BatchItem it{i, y0, std::min(TY, Y - y0), st};
+            units.back().items.push_back(it);
+            units.back().cost += cost(it);
+          }
+        total += units.back().cost;
+      }
+      std::vector<Unit> pieces;
+      for (Unit& u : units) {
+        if (u.cost * 64 <= total) {
+          pieces.push_back(std::move(u));
+          continue;
+        }
+        pieces.push_back(Unit{0, {}});
+        for (const BatchItem& it : u.items) {
+          if (pieces.back().cost * 64 > total) pieces.push_back(Unit{0, {}});
+          pieces.back().items.push_back(it);
+          pieces.back().cost += cost(it);
+        }
+      }
+      // the largest first, each to the XCD with the least so far
+      std::stable_sort(pieces.begin(), pieces.end(),
+                       [](const Unit& a, const Unit& b) { return a.cost > b.cost; });
+      Unit xcd[kXcds];
+      for (Unit& x : xcd) x.cost = 0;
+      for (const Unit& u : pieces) {
+        Unit* least = std::min_element(
+            xcd, xcd + kXcds, [](const Unit& a, const Unit& b) { return a.cost < b.cost; });
+        least->cost += u.cost;
+        least->items.insert(least->items.end(), u.items.begin(), u.items.end());
+      }
+      size_t longest = 0;
+      for (Unit& x : xcd) {
+        std::stable_sort(x.items.begin(), x.items.end(),
+                         [&](const BatchItem& a, const BatchItem& b) {
+                           return cost(a) > cost(b);
+                         });
+        longest = std::max(longest, x.items.size());
+      }
+      std::vector<BatchItem> items;
+      for (size_t q = 0; q < longest; q += kWaves)
+        for (const Unit& x : xcd)
+          for (size_t w = q; w < q + kWaves; ++w)
+            items.push_back(w < x.items.size() ? x.items[w] : BatchItem{0, 0, 0, 0});
       if (d_items[k - 1]) (void)hipFree(d_items[k - 1]);
       d_items[k - 1] = nullptr;
       nitems[k - 1] = (int)items.size();
@@ -376,6 +469,7 @@ int sps_fd_batch_create(const sps_fd_desc* descs, int count,
     return fail(SPS_E_HIP);
   }
   if (sps_fd_batch_set_energy(b, nullptr) != SPS_OK) return fail(SPS_E_HIP);
+  b->choose_rows();
   int rc = b->build_items();
   if (rc != SPS_OK) return fail(rc);
   // persistent grid: as many workgroups as are resident on the device at once

@@ -17,6 +17,7 @@
 #include "lanes.hpp"
 #include "multi.hpp"
 #include "plan.hpp"
+#include "shape.hpp"
 #include "textio.hpp"
 
 namespace sps {
@@ -342,6 +343,14 @@ struct MultiLaunch {
     return vec == 16 / (int)sizeof(T)
                ? launch_multi_v<T, 16 / sizeof(T), K, R, LIN, PC>(in, out, X, Y, TY, c, s)
                : launch_multi_v<T, 8 / sizeof(T), K, R, LIN, PC>(in, out, X, Y, TY, c, s);
+  }
+};
+
+// Whether c runs an instance with known classes.
+struct KnownClasses {
+  template <int R, int LIN, class PC>
+  bool run() const {
+    return PC::a[0] != kPolyAny;
   }
 };
 
@@ -1012,26 +1021,32 @@ int sps_fdm_create(const sps_fdm_desc* desc, sps_fdm_plan** out) {
   if (p->path == SPS_PATH_FUSED) {
     make_mfused_coef(*desc, p->low, p->fc32);
     make_mfused_coef(*desc, p->low, p->fc64);
+    // launch shape before any tuning (shape.hpp)
+    const int R = p->low.radius;
+    StreamShape s;
     if (desc->dim == 3) {
-      // two fields per stage: radius one fuses 2 steps, radius two 1; the
-      // z-chunk splits the grid into about one round of resident waves
-      p->K = p->low.radius == 1 ? 2 : 1;
-      p->TY = p->esize == 8 ? 4 : 8;  // FP64 8-row rings exceed 256 VGPRs
-      p->VEC = 1;
-      const int halo = p->low.radius * p->K;
-      const int64_t per_chunk =
-          (int64_t)((desc->n[0] + 63 - 2 * halo) / (64 - 2 * halo)) *
-          ((desc->n[1] + p->TY - 1) / p->TY);
-      const int64_t m = std::max<int64_t>(1, 2048 / per_chunk);
-      p->TZ = (int)std::min<int64_t>(
-          1024, std::max<int64_t>(16, (desc->n[2] + m - 1) / m));
+      // radius one fuses up to 2 steps, radius two 1 (FP64 8-row rings exceed
+      // 256 VGPRs at two steps)
+      static const Stream3DCand r1[2][3] = {
+          {{2, 4, 0.80}, {2, 8, 1.30}, {1, 4, 0.51}},
+          {{2, 4, 0.95}, {1, 8, 1.10}, {1, 4, 0.60}}};
+      static const Stream3DCand r2[2][2] = {{{1, 4, 0.60}, {1, 8, 0.95}},
+                                            {{1, 4, 0.75}, {1, 8, 1.40}}};
+      const int w = p->esize == 8;
+      s = stream_shape3d(desc->n[0], desc->n[1], desc->n[2], R, (int)p->esize, 2,
+                         R == 1 ? r1[w] : r2[w], R == 1 ? 3 : 2, 1.2);
+    } else if (with_classes(p->fc64, KnownClasses{})) {
+      s = stream_shape2d(desc->n[0], desc->n[1], 4, R, (int)p->esize);
     } else {
-      p->K = p->low.radius == 1 ? 4 : 2;
-      p->TY = 32;
-      // 8-byte lanes: the 16-byte variant holds twice the rows in registers
-      // and measured slower at every launch shape on 4096^2 FP32
-      p->VEC = 8 / (int)p->esize;
+      // stages with a branch per polynomial: fewer steps, and three waves to
+      // cover a row's latency; 8-byte lanes (the 16-byte variant holds twice
+      // the rows in registers)
+      s = stream_shape2d(desc->n[0], desc->n[1], R == 1 ? 4 : 2, R, (int)p->esize, 3.0);
     }
+    p->K = s.steps;
+    p->TY = s.rows;
+    p->VEC = s.vec;
+    if (desc->dim == 3) p->TZ = s.planes;
   }
   hipError_t e = hipStreamCreateWithFlags(&p->own_stream, hipStreamNonBlocking);
   if (e != hipSuccess) {

@@ -1,11 +1,10 @@
 // plan.hpp - the single-field plan behind sps_fd_plan*.
 #pragma once
 
-#include <algorithm>
-
 #include "common.hpp"
 #include "energy.hpp"
 #include "fused.hpp"
+#include "shape.hpp"
 
 namespace sps {
 void set_error(const char* fmt, ...);
@@ -66,32 +65,30 @@ struct sps_fd_plan {
   int step(int nsteps);
   void drop_graphs();
 
-  // Launch shape before any tuning.  2D: the best of a sweep of steps per
-  // launch {1..4} x rows per chunk x lane width on Model B 4096^2 (FP32:
-  // 4 x 32 rows, 2 values per lane; FP64: 4 x 64).  3D: two steps per launch
-  // (FP32: 12 rows per wave, two waves per SIMD at 254 VGPRs; FP64: 4 rows,
-  // one wave per SIMD) with the z-chunk height that splits the grid into as
-  // few rounds of resident waves as possible.
+  // Launch shape before any tuning (shape.hpp).  2D: four steps per launch,
+  // the best at every size measured.  3D: t of the (steps, rows) shapes as
+  // fitted over 32^3 .. 256^3 and uneven boxes (FP32 12 rows at two steps fill
+  // two waves per SIMD; FP64 rings of two steps hold four rows).
   void choose_default_shape() {
-    if (d.dim == 3) {
-      K = 2;
-      TY = d.dtype == SPS_F32 ? 12 : 4;
-      const int slots = d.dtype == SPS_F32 ? 2048 : 1024;  // resident waves
-      const int halo = 2 * K;  // lanes per side at radius two
-      const int64_t per_chunk = (int64_t)((d.n[0] + 63 - 2 * halo) / (64 - 2 * halo)) *
-                                ((d.n[1] + TY - 1) / TY);
-      const int64_t m = std::max<int64_t>(1, slots / per_chunk);
-      TZ = (int)std::min<int64_t>(1024, std::max<int64_t>(16, (d.n[2] + m - 1) / m));
+    const int R = fc64.radius;
+    sps::StreamShape s;
+    if (d.dim == 2) {
+      s = sps::stream_shape2d(d.n[0], d.n[1], 4, R, (int)esize);
     } else if (d.dtype == SPS_F32) {
-      K = 4;
-      TY = 32;
+      static const sps::Stream3DCand c[2][4] = {
+          {{2, 4, 0.258}, {2, 6, 0.333}, {2, 8, 0.433}, {2, 12, 0.603}},
+          {{2, 4, 0.422}, {2, 6, 0.513}, {2, 8, 0.652}, {2, 12, 0.836}}};
+      s = sps::stream_shape3d(d.n[0], d.n[1], d.n[2], R, 4, 1, c[R - 1], 4, 1.4);
     } else {
-      K = 4;
-      TY = 64;
+      static const sps::Stream3DCand c[2][4] = {
+          {{2, 4, 0.418}, {1, 4, 0.366}, {1, 8, 0.583}, {1, 12, 0.779}},
+          {{2, 4, 0.837}, {1, 4, 0.404}, {1, 8, 0.681}, {1, 12, 0.949}}};
+      s = sps::stream_shape3d(d.n[0], d.n[1], d.n[2], R, 8, 1, c[R - 1], 4, 1.1);
     }
-    // FP32 2D: 8-byte lanes (2 values) won the shape sweep; FP64: 16-byte
-    VEC = (d.dim == 2 && d.dtype == SPS_F32) ? 8 / (int)esize : 16 / (int)esize;
-    if (d.dim == 2 && d.n[0] % VEC != 0) VEC = 8 / (int)esize;
+    K = s.steps;
+    TY = s.rows;
+    TZ = d.dim == 3 ? s.planes : 64;
+    VEC = d.dim == 2 ? s.vec : 16 / (int)esize;
   }
 
   int allocate() {
