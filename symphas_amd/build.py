@@ -22,6 +22,7 @@ LIB = LIBDIR / "libsps_fd.so"
 SOURCES = {
     "api.hip": [],
     "ref_kernels.hip": ["-ffp-contract=off"],
+    "ref3d.hip": ["-ffp-contract=off"],
     "fused2d.hip": [],
     "fused3d.hip": [],
     "reduce.hip": [],

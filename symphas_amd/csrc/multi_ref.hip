@@ -7,6 +7,8 @@
 // reference's stencil groupings, a monomial operand evaluated at each stencil
 // point as its temporary grid would hold it) and writes psi_f + dt * rhs_f.
 // Periodic neighbours are found by wrapping coordinates.
+#include <cstring>
+
 #include "multi.hpp"
 #include "ref_stream.hpp"
 #include "stencil_ref.hpp"
@@ -246,10 +248,10 @@ struct FormStep {
   __device__ __forceinline__ T lap_operand(const T (&x)[2]) const {
     return mono<kOps.a[d], kOps.b[d]>(x);
   }
-  template <int S>
-  __device__ __forceinline__ void rhs(
-      const RsWindow<T> (&F)[2], const RsWindow<T> (&D)[NLAP > 0 ? NLAP : 1],
-      const T (&x)[2], T (&r)[2]) const {
+  template <class A>
+  __device__ __forceinline__ void rhs(const A (&F)[2],
+                                      const A (&D)[NLAP > 0 ? NLAP : 1],
+                                      const T (&x)[2], T (&r)[2]) const {
     static_for<0, 2>([&](auto ec) {
       constexpr int e = decltype(ec)::value;
       T acc = T(0);
@@ -261,11 +263,11 @@ struct FormStep {
           v = mono<m.a, m.b>(x);
         } else if constexpr (m.op == SPS_OP_BILAP) {
           static_assert(m.a + m.b == 1, "the bilaplacian of a field");
-          v = rs_bilap2<T, B>(RsAcc<T, S>{F[m.b]}, divh4);
+          v = rs_bilap<B>(F[m.b], divh4);
         } else if constexpr (m.a + m.b == 1) {
-          v = rs_lap2<T, L>(RsAcc<T, S>{F[m.b]}, divh2);
+          v = rs_lap<L>(F[m.b], divh2);
         } else {
-          v = rs_lap2<T, L>(RsAcc<T, S>{D[kOps.find(m.a, m.b)]}, divh2);
+          v = rs_lap<L>(D[kOps.find(m.a, m.b)], divh2);
         }
         acc = t == 0 ? coeff[e][t] * v : acc + coeff[e][t] * v;
       });
@@ -291,6 +293,7 @@ template <typename T, const MForm& FORM, int L, int B>
 void launch_form_lb(const MRefParams<T>& p, hipStream_t s) {
   FormStep<T, FORM, L, B> step;
   RsFields<T, 2> g;
+  std::memset(&g, 0, sizeof(g));
   for (int e = 0; e < 2; ++e) {
     for (int t = 0; t < 5; ++t)
       step.coeff[e][t] = t < FORM.n[e] ? p.terms[e][t].coeff : T(0);
@@ -302,7 +305,11 @@ void launch_form_lb(const MRefParams<T>& p, hipStream_t s) {
   step.dt = p.dt;
   g.X = p.n[0];
   g.Y = p.n[1];
-  launch_ref_stream2d(g, step, s);
+  g.Z = p.n[2];
+  if constexpr (L == 5 || L == 9)
+    launch_ref_stream2d(g, step, s);
+  else  // FP64 rings of two fields hold two rows
+    launch_ref_stream3d<T, sizeof(T) == 8 ? 2 : 4>(g, step, s);
 }
 
 template <typename T, const MForm& FORM, int L>
@@ -316,9 +323,18 @@ void launch_form_l(const MRefParams<T>& p, hipStream_t s) {
   }
 }
 
+// 2D: every stencil; 3D: the 7- and 15-point laplacians, the 25-point
+// bilaplacian.
 template <typename T, const MForm& FORM>
-bool launch_form(const MRefParams<T>& p, hipStream_t s) {
+bool launch_form(const MRefParams<T>& p, int dim, hipStream_t s) {
   if (!is_form(p, FORM)) return false;
+  if (dim == 3) {
+    if ((p.L != 7 && p.L != 15) || (form_has(FORM, SPS_OP_BILAP) && p.B != 25))
+      return false;
+    if (p.L == 7) launch_form_lb<T, FORM, 7, 25>(p, s);
+    else launch_form_lb<T, FORM, 15, 25>(p, s);
+    return true;
+  }
   if (p.L == 5) launch_form_l<T, FORM, 5>(p, s);
   else launch_form_l<T, FORM, 9>(p, s);
   return true;
@@ -328,9 +344,9 @@ bool launch_form(const MRefParams<T>& p, hipStream_t s) {
 
 template <typename T>
 int launch_ref_multi(const MRefParams<T>& p, int dim, hipStream_t stream) {
-  if (dim == 2 && (launch_form<T, kModelCForm>(p, stream) ||
-                   launch_form<T, kGrayScottForm>(p, stream) ||
-                   launch_form<T, kTuringForm>(p, stream)))
+  if (launch_form<T, kModelCForm>(p, dim, stream) ||
+      launch_form<T, kGrayScottForm>(p, dim, stream) ||
+      launch_form<T, kTuringForm>(p, dim, stream))
     return SPS_OK;
   dim3 block(64, 4, 1);
   dim3 grid((p.n[0] + 63) / 64, (p.n[1] + 3) / 4, dim == 3 ? p.n[2] : 1);
