@@ -67,6 +67,13 @@ int sps_nn_conv3x3_wgrad(const void* x, const void* dpre, int n, int h, int w,
                          int cin, int cout, float* dweight, float* workspace,
                          size_t ws_floats, void* stream);
 
+/* The same with the bias gradient, dbias[k] += sum_{n,h,w} dpre[n,h,w,k], from
+ * the same read of dpre (dbias NULL: the weight gradient alone). */
+int sps_nn_conv3x3_wgrad_bias(const void* x, const void* dpre, int n, int h,
+                              int w, int cin, int cout, float* dweight,
+                              float* dbias, float* workspace, size_t ws_floats,
+                              void* stream);
+
 /* First layer, one FP32 input channel:
  *   pre[n,h,w,k] = bias[k] + sum_t x[n, shift_t(h,w)] * weight[t][k],
  *   y = act(pre) (BF16), weight [9][cout] FP32, cout % 8 == 0, cout <= 64. */

@@ -15,8 +15,8 @@
 // consecutive output channels of a pixel per lane (8 bytes).
 //
 // The weight gradient reduces over pixels, which are strided in NHWC, so it
-// stages a 32-pixel row chunk of dpre and the three shifted input rows in LDS
-// and gathers the fragments from there.
+// stages a block of pixels of dpre and of the input with its halo in LDS and
+// reads the fragments from there transposed (ds_read_b64_tr_b16).
 #include <algorithm>
 #include <cstdint>
 #include <initializer_list>
@@ -451,7 +451,220 @@ __global__ __launch_bounds__(256) void conv_fwd_tile(
   }
 }
 
-// Weight gradient: tile KT x CT of [k][c] for all 9 taps, reduction over
+// Weight gradient (and bias gradient) on blocks of pixels: a workgroup owns a
+// KT x CT tile of [k][c] for all 9 taps and walks chunks of RC rows x WC
+// columns.  Per chunk dpre and the input with its 1-pixel periodic halo are
+// copied to LDS (two buffers, the next chunk's loads in flight during this
+// one's products).  Both operands need consecutive pixels of one channel per
+// lane while LDS rows are consecutive channels of one pixel:
+// ds_read_b64_tr_b16 transposes 4 pixels x 16 channels per 16 lanes.  The
+// three horizontal taps come from one read of 12 pixels, shifted in registers.
+// Each of the 8 waves holds a 32 x 32 part of the tile (144 accumulators) and
+// the WP waves of a part split the chunk's pixels; their sums are added in
+// order at the end.  Rows are padded so that the 4 pixels of a read fall in
+// different banks.
+// The form that gathered fragments with 2-byte LDS reads and staged 32 pixels
+// at a time took (batch 32) 128 us for 32->32 at 256^2 and 94 on average for
+// the layers of 64 channels and more; this one 75 and 40 (with the sum over
+// workgroups 470 and 600 TFLOP/s), the bias gradient included, which was a
+// pass over dpre of its own (37 us on average).
+typedef short i16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 read_tr(const uint16_t* p) {
+  return __builtin_bit_cast(
+      uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                 (__attribute__((address_space(3))) i16x4*)p));
+}
+
+template <int KT, int CT, int WC>
+struct WgradTile {
+  static constexpr int kThreads = 512;
+  static constexpr int WK = KT / 32, WCT = CT / 32;  // parts of the tile
+  static constexpr int WP = 8 / (WK * WCT);          // waves of a part
+  static constexpr int PX = WP == 8 ? 256 : 128;     // pixels of a chunk
+  static constexpr int KS = PX / 32 / WP;            // MFMA steps of a wave
+  static constexpr int RC = PX / WC;                 // rows of a chunk
+  static constexpr int XC = WC + 4;  // halo, and 2 columns only read past it
+  static constexpr int SD = KT + (KT == 64 ? 8 : 16);  // row strides
+  static constexpr int SX = CT + (CT == 64 ? 8 : 16);
+  static constexpr int kDy = PX * SD, kX = (RC + 2) * XC * SX;
+  static constexpr int kBuf = kDy + kX;
+};
+
+template <int KT, int CT, int WC>
+__global__ __launch_bounds__(512) void conv_wgrad_tile(
+    const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy, int H,
+    int W, int C, int K, float* __restrict__ part, int64_t slice, int nchunks,
+    int per, int with_bias) {
+  using G = WgradTile<KT, CT, WC>;
+  constexpr int NT = G::kThreads;
+  __shared__ __align__(16) uint16_t lds[2 * G::kBuf];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wk = wave % G::WK, wc = wave / G::WK % G::WCT,
+            wp = wave / (G::WK * G::WCT);
+  const int c0 = blockIdx.x * CT, k0 = blockIdx.y * KT;
+  const int cblocks = W / WC, rblocks = H / G::RC;
+
+  constexpr int DP = G::PX * KT / 8, XP = (G::RC + 2) * (WC + 2) * CT / 8;
+  constexpr int ND = (DP + NT - 1) / NT, NX = (XP + NT - 1) / NT;
+  u32x4 rd[ND], rx[NX];
+  auto fetch = [&](int ch) {
+    const int cb = ch % cblocks, t = ch / cblocks;
+    const int h0 = t % rblocks * G::RC, n = t / rblocks, w0 = cb * WC;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const int e = threadIdx.x + NT * i;
+      const int px = e / (KT / 8), k = e % (KT / 8) * 8;
+      if (DP % NT == 0 || e < DP)
+        rd[i] = *reinterpret_cast<const u32x4*>(
+            dy + ((int64_t)(n * H + h0 + px / WC) * W + w0 + px % WC) * K + k0 + k);
+    }
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int e = threadIdx.x + NT * i;
+      const int px = e / (CT / 8), c = e % (CT / 8) * 8;
+      const int r = px / (WC + 2), q = px % (WC + 2);
+      if (XP % NT == 0 || e < XP)
+        rx[i] = *reinterpret_cast<const u32x4*>(
+            x + ((int64_t)(n * H + wrapi(h0 + r - 1, H)) * W + wrapi(w0 + q - 1, W)) * C +
+            c0 + c);
+    }
+  };
+  auto put = [&](uint16_t* b) {
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const int e = threadIdx.x + NT * i;
+      const int px = e / (KT / 8), k = e % (KT / 8) * 8;
+      if (DP % NT == 0 || e < DP) *reinterpret_cast<u32x4*>(b + px * G::SD + k) = rd[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int e = threadIdx.x + NT * i;
+      const int px = e / (CT / 8), c = e % (CT / 8) * 8;
+      const int r = px / (WC + 2), q = px % (WC + 2);
+      if (XP % NT == 0 || e < XP)
+        *reinterpret_cast<u32x4*>(b + G::kDy + (r * G::XC + q) * G::SX + c) = rx[i];
+    }
+  };
+
+  f32x4v acc[9][2][2], accb[2];
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[t][a][b] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  accb[0] = accb[1] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  const bool bias_wave = with_bias && blockIdx.x == 0 && wc == 0;
+  constexpr uint32_t kOnes = 0x3f803f80u;  // two BF16 ones
+  const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{kOnes, kOnes, kOnes, kOnes});
+
+  const int first = blockIdx.z * per, last = min(nchunks, first + per);
+  if (first < last) {
+    fetch(first);
+    put(lds);
+  }
+  __syncthreads();
+  for (int ch = first; ch < last; ++ch) {
+    if (ch + 1 < last) fetch(ch + 1);
+    const uint16_t* b = lds + ((ch - first) & 1) * G::kBuf;
+#pragma unroll
+    for (int ks = 0; ks < G::KS; ++ks) {
+      // this lane group's 8 pixels, one row's
+      const int px = 32 * (wp * G::KS + ks) + 8 * (lane >> 4);
+      const int row = px / WC, col = px % WC;
+      const int tp = (lane & 15) >> 2, tc4 = 4 * (lane & 3);
+      bf16x8 a[2];
+#pragma unroll
+      for (int tk = 0; tk < 2; ++tk) {
+        const uint16_t* q = b + (px + tp) * G::SD + 32 * wk + 16 * tk + tc4;
+        const uint2 u = read_tr(q), v = read_tr(q + 4 * G::SD);
+        a[tk] = __builtin_bit_cast(bf16x8, u32x4{u.x, u.y, v.x, v.y});
+      }
+      if (bias_wave) {
+#pragma unroll
+        for (int tk = 0; tk < 2; ++tk)
+          accb[tk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tk], ones, accb[tk], 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int tc = 0; tc < 2; ++tc) {
+          const uint16_t* q = b + G::kDy + ((row + r) * G::XC + col + tp) * G::SX +
+                              32 * wc + 16 * tc + tc4;
+          const uint2 u = read_tr(q), v = read_tr(q + 4 * G::SX), w = read_tr(q + 8 * G::SX);
+          const uint32_t d[5] = {u.x, u.y, v.x, v.y, w.x};  // pixels 0 .. 9
+          u32x4 f[3];
+          f[0] = u32x4{d[0], d[1], d[2], d[3]};
+          f[2] = u32x4{d[1], d[2], d[3], d[4]};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) f[1][i] = __builtin_amdgcn_alignbit(d[i + 1], d[i], 16);
+#pragma unroll
+          for (int s3 = 0; s3 < 3; ++s3)
+#pragma unroll
+            for (int tk = 0; tk < 2; ++tk)
+              acc[3 * r + s3][tk][tc] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  a[tk], __builtin_bit_cast(bf16x8, f[s3]), acc[3 * r + s3][tk][tc], 0, 0, 0);
+        }
+    }
+    if (ch + 1 < last) put(lds + ((ch + 1 - first) & 1) * G::kBuf);
+    __syncthreads();
+  }
+
+  // add the WP waves of each part in order through LDS, a tap row at a time,
+  // then the bias sums
+  if constexpr (G::WP > 1) {
+    constexpr int PARTS = G::WK * G::WCT;
+    static_assert((G::WP - 1) * PARTS * 64 * 12 * 16 <= 2 * G::kBuf * 2, "fits");
+    f32x4v* red = reinterpret_cast<f32x4v*>(lds);
+    auto slot = [&](int p) { return red + ((p - 1) * PARTS + wk + G::WK * wc) * 12 * 64 + lane; };
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (wp > 0) {
+        f32x4v* o = slot(wp);
+#pragma unroll
+        for (int i = 0; i < (r < 3 ? 12 : 2); ++i)
+          o[64 * i] = r < 3 ? acc[3 * (r % 3) + i / 4][i / 2 % 2][i % 2] : accb[i % 2];
+      }
+      __syncthreads();
+      if (wp == 0) {
+        for (int p = 1; p < G::WP; ++p) {
+          const f32x4v* o = slot(p);
+#pragma unroll
+          for (int i = 0; i < (r < 3 ? 12 : 2); ++i) {
+            if (r < 3) acc[3 * (r % 3) + i / 4][i / 2 % 2][i % 2] += o[64 * i];
+            else accb[i % 2] += o[64 * i];
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+  if (wp > 0) return;
+  // this workgroup's partial sums (zeros if it had no chunk)
+  float* dw = part + (int64_t)blockIdx.z * slice;
+#pragma unroll
+  for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+    for (int tk = 0; tk < 2; ++tk)
+#pragma unroll
+      for (int tc = 0; tc < 2; ++tc)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int k = k0 + 32 * wk + 16 * tk + 4 * (lane >> 4) + i;
+          const int c = c0 + 32 * wc + 16 * tc + (lane & 15);
+          dw[((int64_t)tap * K + k) * C + c] = acc[tap][tk][tc][i];
+        }
+  if (bias_wave && (lane & 15) == 0) {
+#pragma unroll
+    for (int tk = 0; tk < 2; ++tk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        dw[(int64_t)9 * K * C + k0 + 32 * wk + 16 * tk + 4 * (lane >> 4) + i] = accb[tk][i];
+  }
+}
+
+// The general weight gradient, for images that do not split into whole chunks
+// of the tiled one: tile KT x CT of [k][c] for all 9 taps, reduction over
 // 32-pixel row chunks staged in LDS.  Wave w owns k rows [w%2 * KT/2, +KT/2)
 // and c columns [w/2 * CT/2, +CT/2).
 // ROWS: chunks are 32-pixel pieces of one row (w % 32 == 0) and the three
@@ -460,8 +673,8 @@ __global__ __launch_bounds__(256) void conv_fwd_tile(
 template <int KT, int CT, bool ROWS>
 __global__ __launch_bounds__(256) void conv_wgrad(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy, int N,
-    int H, int W, int C, int K, float* __restrict__ part, int nchunks,
-    int chunks_per_block) {
+    int H, int W, int C, int K, float* __restrict__ part, int64_t slice,
+    int nchunks, int chunks_per_block) {
   constexpr int TK = KT / 32, TC = CT / 32;  // MFMA tiles per wave
   __shared__ __align__(16) uint16_t sdy[32][KT + 2];
   __shared__ __align__(16) uint16_t sx[ROWS ? 3 : 9][ROWS ? 34 : 32][CT + 2];
@@ -560,7 +773,7 @@ __global__ __launch_bounds__(256) void conv_wgrad(
     }
   }
   // this block's partial sums (zeros if it had no chunk): slice blockIdx.z
-  float* dw = part + (int64_t)blockIdx.z * 9 * K * C;
+  float* dw = part + (int64_t)blockIdx.z * slice;
 #pragma unroll
   for (int tap = 0; tap < 9; ++tap)
 #pragma unroll
@@ -943,14 +1156,30 @@ __global__ __launch_bounds__(256) void sum_partial_groups(float* __restrict__ pa
   }
 }
 
+// The first nw sums go to dw, the others (a bias gradient) to db.
 __global__ __launch_bounds__(256) void add_partials(const float* __restrict__ part,
                                                     int M, int64_t S, int64_t count,
-                                                    float* __restrict__ dw) {
+                                                    float* __restrict__ dw, int64_t nw,
+                                                    float* __restrict__ db) {
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count;
        i += (int64_t)gridDim.x * 256) {
     float s = 0.f;
     for (int m = 0; m < M; ++m) s += part[(int64_t)m * S * count + i];
-    dw[i] += s;
+    if (i < nw) dw[i] += s;
+    else db[i - nw] += s;
+  }
+}
+
+// Bias gradient of the general path: workgroup z sums channels of its pixels.
+__global__ __launch_bounds__(256) void bias_partials(const uint16_t* __restrict__ dy,
+                                                     int64_t npix, int K, int64_t per,
+                                                     float* __restrict__ part,
+                                                     int64_t slice) {
+  const int64_t p0 = blockIdx.x * per, p1 = min(npix, p0 + per);
+  for (int k = threadIdx.x; k < K; k += 256) {
+    float s = 0.f;
+    for (int64_t p = p0; p < p1; ++p) s += bf2f(dy[p * K + k]);
+    part[blockIdx.x * slice + k] = s;
   }
 }
 
@@ -1142,12 +1371,27 @@ struct WgradSplit {
   int64_t count; // floats of one partial gradient
 };
 
-WgradSplit conv_split(int64_t npix, int cin, int cout) {
+// Columns of the tiled weight gradient's chunks (32, 16 or 8, the widest whose
+// chunks cover the image exactly); 0 for the general kernel.  *px: pixels of a
+// chunk.
+int wgrad_cols(int h, int w, int cin, int cout, int* px) {
+  *px = cin % 64 != 0 && cout % 64 != 0 ? 256 : 128;
+  for (int wc : {32, 16, 8})
+    if (w % wc == 0 && h % (*px / wc) == 0) return wc;
+  *px = 32;
+  return 0;
+}
+
+WgradSplit conv_split(int n, int h, int w, int cin, int cout) {
   const int kt = cout % 64 == 0 ? 64 : 32, ct = cin % 64 == 0 ? 64 : 32;
-  const int64_t nchunks = npix / 32;
+  const int64_t npix = (int64_t)n * h * w;
   const int64_t count = (int64_t)9 * cin * cout;
   const int64_t tiles = (int64_t)(cin / ct) * (cout / kt);
-  int64_t nz = (2048 + tiles - 1) / tiles;
+  int px;
+  // the tiled kernel's LDS leaves one workgroup per CU: one round of 256
+  const bool tiled = wgrad_cols(h, w, cin, cout, &px) != 0;
+  const int64_t nchunks = npix / px;
+  int64_t nz = tiled ? 256 / tiles : (2048 + tiles - 1) / tiles;
   nz = std::min<int64_t>(nz, std::max<int64_t>(1, kPartFloats / count));
   nz = std::max<int64_t>(1, std::min<int64_t>(nz, nchunks));
   const int64_t per = (nchunks + nz - 1) / nz;
@@ -1172,7 +1416,8 @@ WgradSplit out1_split(int n, int h, int w, int c) {
 }
 
 // The workspace's partials are consumed (summed in place).
-int add_parts(float* part, const WgradSplit& sp, float* dw, hipStream_t s) {
+int add_parts(float* part, const WgradSplit& sp, float* dw, hipStream_t s,
+              int64_t nw = -1, float* db = nullptr) {
   constexpr int kGroup = 32;
   int M = sp.blocks;
   int64_t S = 1;
@@ -1183,7 +1428,8 @@ int add_parts(float* part, const WgradSplit& sp, float* dw, hipStream_t s) {
     M = (int)ng;
     S *= kGroup;
   }
-  add_partials<<<grid_for(sp.count), 256, 0, s>>>(part, M, S, sp.count, dw);
+  add_partials<<<grid_for(sp.count), 256, 0, s>>>(part, M, S, sp.count, dw,
+                                                  nw < 0 ? sp.count : nw, db);
   return launch_ok("weight-gradient partial sum");
 }
 
@@ -1283,8 +1529,10 @@ size_t sps_nn_wgrad_workspace(int kind, int n, int h, int w, int cin,
   if (n < 1 || h < 1 || w < 1 || cin < 1 || cout < 1) return 0;
   const int64_t np = (int64_t)n * h * w;
   WgradSplit sp{0, 0, 0};
-  if (kind == SPS_NN_WGRAD_CONV) sp = conv_split(np, cin, cout);
-  else if (kind == SPS_NN_WGRAD_IN1) sp = chunk_split(np, (int64_t)9 * cout);
+  if (kind == SPS_NN_WGRAD_CONV) {
+    sp = conv_split(n, h, w, cin, cout);
+    sp.count += cout;  // the bias gradient
+  } else if (kind == SPS_NN_WGRAD_IN1) sp = chunk_split(np, (int64_t)9 * cout);
   else if (kind == SPS_NN_WGRAD_OUT1) sp = out1_split(n, h, w, cin);
   return (size_t)((int64_t)sp.blocks * sp.count);
 }
@@ -1292,6 +1540,14 @@ size_t sps_nn_wgrad_workspace(int kind, int n, int h, int w, int cin,
 int sps_nn_conv3x3_wgrad(const void* x, const void* dpre, int n, int h, int w,
                          int cin, int cout, float* dweight, float* workspace,
                          size_t ws_floats, void* stream) {
+  return sps_nn_conv3x3_wgrad_bias(x, dpre, n, h, w, cin, cout, dweight, nullptr,
+                                   workspace, ws_floats, stream);
+}
+
+int sps_nn_conv3x3_wgrad_bias(const void* x, const void* dpre, int n, int h,
+                              int w, int cin, int cout, float* dweight,
+                              float* dbias, float* workspace, size_t ws_floats,
+                              void* stream) {
   const int64_t npix = (int64_t)n * h * w;
   if (!x || !dpre || !dweight || n < 1 || h < 1 || w < 1 || npix % 32 ||
       npix > (int64_t)1 << 30 || cin % 32 || cout % 32 || cin < 32 ||
@@ -1299,10 +1555,15 @@ int sps_nn_conv3x3_wgrad(const void* x, const void* dpre, int n, int h, int w,
     set_error("sps_nn_conv3x3_wgrad: need n*h*w, cin, cout multiples of 32");
     return SPS_E_INVALID;
   }
-  const WgradSplit sp = conv_split(npix, cin, cout);
+  WgradSplit sp = conv_split(n, h, w, cin, cout);
+  const int64_t nw = sp.count;
+  if (dbias) sp.count += cout;
   SPS_TRY(check_ws("sps_nn_conv3x3_wgrad", sp, workspace, ws_floats));
-  const bool rows = w % 32 == 0;
-  const int nchunks = (int)(npix / 32);
+  int px;
+  // 16-byte loads in either kernel; the general one takes any alignment that
+  // its own loads do
+  const int wc = wgrad_cols(h, w, cin, cout, &px);
+  const int nchunks = (int)(npix / px);
   const int per = sp.per;
   const int kt = cout % 64 == 0 ? 64 : 32;
   const int ct = cin % 64 == 0 ? 64 : 32;
@@ -1310,11 +1571,21 @@ int sps_nn_conv3x3_wgrad(const void* x, const void* dpre, int n, int h, int w,
   hipStream_t s = (hipStream_t)stream;
   const uint16_t* xx = (const uint16_t*)x;
   const uint16_t* dd = (const uint16_t*)dpre;
+#define SPS_WGRAD_TILE(KT_, CT_, WC_)                                         \
+  conv_wgrad_tile<KT_, CT_, WC_><<<grid, 512, 0, s>>>(                        \
+      xx, dd, h, w, cin, cout, workspace, sp.count, nchunks, per, dbias != nullptr)
 #define SPS_WGRAD(KT_, CT_)                                                   \
-  (rows ? (conv_wgrad<KT_, CT_, true><<<grid, 256, 0, s>>>(                   \
-               xx, dd, n, h, w, cin, cout, workspace, nchunks, per), 0)      \
-        : (conv_wgrad<KT_, CT_, false><<<grid, 256, 0, s>>>(                  \
-               xx, dd, n, h, w, cin, cout, workspace, nchunks, per), 0))
+  do {                                                                        \
+    if (wc == 32) SPS_WGRAD_TILE(KT_, CT_, 32);                               \
+    else if (wc == 16) SPS_WGRAD_TILE(KT_, CT_, 16);                          \
+    else if (wc == 8) SPS_WGRAD_TILE(KT_, CT_, 8);                            \
+    else if (w % 32 == 0)                                                     \
+      conv_wgrad<KT_, CT_, true><<<grid, 256, 0, s>>>(                        \
+          xx, dd, n, h, w, cin, cout, workspace, sp.count, nchunks, per);     \
+    else                                                                      \
+      conv_wgrad<KT_, CT_, false><<<grid, 256, 0, s>>>(                       \
+          xx, dd, n, h, w, cin, cout, workspace, sp.count, nchunks, per);     \
+  } while (0)
   if (kt == 64 && ct == 64)
     SPS_WGRAD(64, 64);
   else if (kt == 64)
@@ -1324,8 +1595,14 @@ int sps_nn_conv3x3_wgrad(const void* x, const void* dpre, int n, int h, int w,
   else
     SPS_WGRAD(32, 32);
 #undef SPS_WGRAD
+#undef SPS_WGRAD_TILE
   SPS_TRY(launch_ok("sps_nn_conv3x3_wgrad"));
-  return add_parts(workspace, sp, dweight, s);
+  if (dbias && !wc) {
+    bias_partials<<<(unsigned)sp.blocks, 256, 0, s>>>(
+        dd, npix, cout, (int64_t)per * px, workspace + nw, sp.count);
+    SPS_TRY(launch_ok("sps_nn_conv3x3_wgrad_bias"));
+  }
+  return add_parts(workspace, sp, dweight, s, nw, dbias);
 }
 
 int sps_nn_conv3x3_in1(const float* x, int n, int h, int w,

@@ -76,6 +76,17 @@ def conv3x3_wgrad_raw(x, dpre, K):
     return dw
 
 
+def conv3x3_wgrad_bias_raw(x, dpre, K):
+    """The weight gradient and the bias gradient from one read of dpre."""
+    N, H, W, C = x.shape
+    g = torch.zeros(9 * K * C + K, device=x.device, dtype=torch.float32)
+    dw, db = g[:9 * K * C].view(9, K, C), g[9 * K * C:]
+    ws = wgrad_workspace(WGRAD_CONV, N, H, W, C, K, x.device)
+    _check(_lib().sps_nn_conv3x3_wgrad_bias(_ptr(x), _ptr(dpre), N, H, W, C, K, _ptr(dw), _ptr(db),
+                                            _ptr(ws), ws.numel(), _stream()))
+    return dw, db
+
+
 def silu_bwd_raw(dy, pre):
     dx = torch.empty_like(dy)
     _check(_lib().sps_nn_silu_bwd(_ptr(dy), _ptr(pre), _ptr(dx), dy.numel(), _stream()))
@@ -127,9 +138,8 @@ class _Conv(torch.autograd.Function):
         K, C = w.shape[1], w.shape[2]
         wb = flip_weights(w.detach()).to(torch.bfloat16)
         dx, _ = conv3x3_raw(dlow, wb, None, ACT_NONE)
-        dw = conv3x3_wgrad_raw(x.contiguous(), dlow, K)
-        # FP32 accumulation straight from the BF16 gradient (no FP32 copy)
-        db = torch.sum(dlow, dim=(0, 1, 2), dtype=torch.float32)
+        # FP32 sums straight from the BF16 gradient
+        dw, db = conv3x3_wgrad_bias_raw(x.contiguous(), dlow, K)
         return dx, dw, db, None, None, dskip, None
 
 

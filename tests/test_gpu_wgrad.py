@@ -1,0 +1,39 @@
+"""The tiled weight gradient and its bias gradient: chunk widths, part shapes,
+remainders over workgroups, against FP64 sums of the same BF16 values."""
+import numpy as np
+import pytest
+import torch
+
+from symphas_amd import nn
+
+pytestmark = pytest.mark.gpu
+
+
+# chunks of 32, 16 and 8 columns; 64 and 32 channel tiles; one chunk, more
+# workgroups than chunks, a last workgroup with fewer; the general kernel
+@pytest.mark.parametrize("N,H,W,C,K", [
+    (1, 4, 32, 64, 64), (3, 8, 64, 64, 64), (2, 8, 16, 64, 64), (5, 16, 8, 64, 64),
+    (1, 8, 32, 32, 32), (2, 16, 48, 32, 32), (1, 32, 24, 32, 32), (17, 24, 32, 32, 32),
+    (1, 4, 32, 32, 64), (2, 8, 16, 32, 128), (1, 16, 40, 32, 64),
+    (1, 4, 32, 64, 32), (2, 8, 48, 128, 32), (3, 16, 8, 64, 96),
+    (2, 32, 32, 256, 128), (4, 64, 64, 64, 128), (1, 64, 320, 64, 64),
+    (2, 4, 8, 64, 32), (1, 2, 32, 32, 64), (4, 3, 8, 32, 32)])
+def test_weight_and_bias_gradients(gpu_lib, N, H, W, C, K):
+    print("[case] wgrad", N, H, W, C, K, flush=True)
+    g = torch.Generator(device="cuda").manual_seed(N * 1000 + W)
+    x = torch.randn(N, H, W, C, device="cuda", generator=g).to(torch.bfloat16)
+    d = torch.randn(N, H, W, K, device="cuda", generator=g).to(torch.bfloat16)
+    dw, db = nn.conv3x3_wgrad_bias_raw(x, d, K)
+    again = nn.conv3x3_wgrad_bias_raw(x, d, K)
+    assert torch.equal(dw, again[0]) and torch.equal(db, again[1])
+    assert torch.equal(dw, nn.conv3x3_wgrad_raw(x, d, K))
+    xd, dd = x.double(), d.double().reshape(-1, K)
+    # FP32 sums of npix products: rounding of a random walk, times a margin
+    tol = 8 * 2.0 ** -24 * np.sqrt(N * H * W)
+    for t in range(9):
+        v = torch.roll(xd, (1 - t // 3, 1 - t % 3), dims=(1, 2)).reshape(-1, C)
+        want = dd.t() @ v
+        scale = float((dd.abs().t() @ v.abs()).max()) / np.sqrt(N * H * W)
+        assert float((dw[t].double() - want).abs().max()) <= tol * scale, t
+    scale = float(dd.abs().sum(0).max()) / np.sqrt(N * H * W)
+    assert float((db.double() - dd.sum(0)).abs().max()) <= tol * scale
