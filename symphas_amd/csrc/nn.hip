@@ -22,6 +22,7 @@
 #include <initializer_list>
 
 #include "common.hpp"
+#include "lanes.hpp"
 #include "../../include/sps_nn.h"
 
 namespace sps {
@@ -241,7 +242,8 @@ __global__ __launch_bounds__(256) void conv_fwd_tile(
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave % WM, wn = wave / WM;
   const int tiles_w = W / kTileCols, tiles_h = H / TH;
-  int t = blockIdx.x;
+  // neighbouring tiles, which share halo pixels, on one XCD
+  int t = xcd_remap(blockIdx.x, gridDim.x);
   const int tw = t % tiles_w;
   t /= tiles_w;
   const int th = t % tiles_h;
@@ -287,13 +289,25 @@ __global__ __launch_bounds__(256) void conv_fwd_tile(
   // NCH > 0: every chunk's loads in flight before the first LDS store
 #pragma unroll
   for (int c = 0; c < NST; ++c) fetch(32 * c, c);
+  // With one chunk and 32 channels per wave the weights of all nine taps fit
+  // the registers (72) at three waves per SIMD: one latency instead of nine
+  // (32->32 at 256^2, batch 64: 190 -> 167 us).
+  constexpr bool ALLW = NCH == 1 && MW == 2;
+  bf16x8 aw[ALLW ? 9 : 1][MW];
+  if constexpr (ALLW) {
+#pragma unroll
+    for (int tap = 0; tap < 9; ++tap)
+#pragma unroll
+      for (int m = 0; m < MW; ++m)
+        aw[tap][m] = load_frag(wt + ((int64_t)tap * K + k0 + 16 * m + (lane & 15)) * C + cq);
+  }
 #pragma unroll
   for (int c = 0; c < NST; ++c) put(c, c);
   for (int ch = 0; ch < nchunks; ++ch) {
     const int buf = NCH ? ch : ch & 1;
     const int c0 = 32 * ch;
-    // weight fragments are loaded one tap ahead of their MFMAs (loading all
-    // nine taps' at once costs the waves a SIMD can hold)
+    // otherwise weight fragments are loaded one tap ahead of their MFMAs
+    // (loading all nine taps' at once costs the waves a SIMD can hold)
     bf16x8 apre[2][MW];
     auto load_a = [&](int tap, bf16x8 (&dst)[MW]) {
 #pragma unroll
@@ -301,7 +315,7 @@ __global__ __launch_bounds__(256) void conv_fwd_tile(
         dst[m] = load_frag(wt + ((int64_t)tap * K + k0 + 16 * m + (lane & 15)) * C +
                            c0 + cq);
     };
-    load_a(0, apre[0]);
+    if constexpr (!ALLW) load_a(0, apre[0]);
     // NCH = 0: tile[buf] written and tile[buf ^ 1] free; NCH > 0: every
     // chunk's tile written
     if (NCH == 0 || ch == 0) __syncthreads();
@@ -311,8 +325,9 @@ __global__ __launch_bounds__(256) void conv_fwd_tile(
     for (int tap = 0; tap < 9; ++tap) {
       const int dr = tap / 3, ds = tap % 3;  // halo-shifted offsets 0..2
       bf16x8 b[NW];
-      if (tap + 1 < 9) load_a(tap + 1, apre[(tap + 1) & 1]);
-      const bf16x8 (&a)[MW] = apre[tap & 1];
+      if constexpr (!ALLW)
+        if (tap + 1 < 9) load_a(tap + 1, apre[(tap + 1) & 1]);
+      const bf16x8 (&a)[MW] = ALLW ? aw[ALLW ? tap : 0] : apre[tap & 1];
 #pragma unroll
       for (int j = 0; j < NW; ++j) {
         const int tr = wn * NW + j + dr;
@@ -448,6 +463,259 @@ __global__ __launch_bounds__(256) void conv_fwd_tile(
           }
       }
     }
+  }
+}
+
+// The plain epilogue of a workgroup: bias and activation on the accumulators,
+// rounded to BF16, then through LDS (pixel stride KB + 8) so that stores are
+// runs of pixels x channels in 16-byte pieces.  acc[m][j] holds channels
+// cl + 16*m .. + 3 of pixel px + 16*j of the tile (16 columns per row).  pre,
+// when asked for, goes the same way first.  (With the FP32 sums staged and
+// activated after the read, twice the LDS bytes, 64->64 took 133 us, not 125.)
+template <int KB, int NPX, int NT, int MW, int NW>
+__device__ __forceinline__ void store_plain(
+    f32x4v (&acc)[MW][NW], uint16_t* stage, int px, int cl,
+    const float* __restrict__ bias, int act, uint16_t* __restrict__ y,
+    uint16_t* __restrict__ pre, int64_t base, int W, int K) {
+  constexpr int S = KB + 8, G = KB / 8;
+  if (bias) {
+#pragma unroll
+    for (int m = 0; m < MW; ++m) {
+      f32x4v b;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) b[i] = bias[cl + 16 * m + i];
+#pragma unroll
+      for (int j = 0; j < NW; ++j) acc[m][j] += b;
+    }
+  }
+  auto pass = [&](uint16_t* out, bool silu_it) {
+    __syncthreads();  // the workgroup is done with what the LDS held
+#pragma unroll
+    for (int m = 0; m < MW; ++m)
+#pragma unroll
+      for (int j = 0; j < NW; ++j) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = silu_it ? silu(acc[m][j][i]) : acc[m][j][i];
+        store4(&stage[(px + 16 * j) * S + cl + 16 * m], v);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int e0 = 0; e0 < NPX * G; e0 += NT) {
+      const int e = e0 + threadIdx.x;
+      if (NPX * G % NT != 0 && e >= NPX * G) break;
+      const int q = e / G, g = e - q * G;
+      *reinterpret_cast<u32x4*>(out + base + ((int64_t)(q / kTileCols) * W + q % kTileCols) * K +
+                                8 * g) =
+          *reinterpret_cast<const u32x4*>(&stage[q * S + 8 * g]);
+    }
+  };
+  if (pre) pass(pre, false);
+  pass(y, act != 0);
+}
+
+// Forward on large tiles, 8 waves: TH = 4*WN rows x 16 columns by KB = 64*WM
+// output channels, each wave 64 channels x 64 pixels.  conv_fwd_tile's waves
+// wait 83% of their time on weights: every wave reads its own fragments from
+// L2 (1.2 GB per call of 256->256 at 32^2, batch 64, for 1.2 MB of weights),
+// and the products keep the matrix cores busy 20% of the time.  Here a
+// workgroup stages the weights of three taps of a 32-channel chunk in LDS, in
+// fragment order, double-buffered like the input tile, with the next group's
+// loads in flight during this group's 48 products per wave, so a weight is
+// read once per 256 or 512 pixels.  Products and sums are those of
+// conv_fwd_tile in the same order.  Bound by LDS reads and barriers now: 40% of
+// the matrix cores' rate at 256 channels.  Measured (us, batch 64, before ->
+// now): 64->64 at 128^2 187 -> 125; 128->128 at 64^2 153 -> 96; 256->256 at
+// 32^2 144 -> 80 (960 TFLOP/s); upsample-add 256->128 149 -> 57, 128->64 181 ->
+// 89.
+template <int WM, int WN, int EPI>
+__global__ __launch_bounds__(512) void conv_fwd_wide(
+    const uint16_t* __restrict__ x, int H, int W, int C,
+    const uint16_t* __restrict__ wt, const float* __restrict__ bias, int K,
+    int act, const uint16_t* __restrict__ skip, uint16_t* __restrict__ y,
+    uint16_t* __restrict__ pre) {
+  static_assert(WM * WN == 8, "8 waves");
+  constexpr int NT = 512, MW = 4, NW = 4;
+  constexpr int TH = NW * WN, KB = 16 * MW * WM;
+  constexpr int TILE = (TH + 2) * kHaloCols;
+  constexpr int TP = TILE * 4, NTP = (TP + NT - 1) / NT;    // tile pieces
+  constexpr int WPC = 3 * KB * 4, NWP = (WPC + NT - 1) / NT;  // weight pieces
+  constexpr int kTile = TILE * kPixStride, kW = 3 * KB * 32;
+  constexpr int SKB = KB + 4;                 // staged pixel stride (FP32)
+  constexpr int PXH = TH * kTileCols / 2;     // pixels of an epilogue pass
+  constexpr int kMain = 2 * (kTile + kW) * 2;
+  constexpr int kEpi = EPI == SPS_NN_EPI_PLAIN ? TH * kTileCols * (KB + 8) * 2 : PXH * SKB * 4;
+  __shared__ __align__(16) unsigned char lds[kMain > kEpi ? kMain : kEpi];
+  uint16_t* const tiles = reinterpret_cast<uint16_t*>(lds);
+  uint16_t* const weights = tiles + 2 * kTile;
+
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave % WM, wn = wave / WM;
+  const int cq = (lane >> 4) * 8;
+  // output-channel blocks of one tile are neighbours, on one XCD
+  const int nkb = K / KB;
+  int t = xcd_remap(blockIdx.x, gridDim.x);
+  const int kb0 = t % nkb * KB;
+  t /= nkb;
+  const int tiles_w = W / kTileCols, tiles_h = H / TH;
+  const int w0 = t % tiles_w * kTileCols;
+  t /= tiles_w;
+  const int h0 = t % tiles_h * TH, n = t / tiles_h;
+
+  int64_t src[NTP];
+#pragma unroll
+  for (int i = 0; i < NTP; ++i) {
+    const int e = threadIdx.x + NT * i, pix = e >> 2, q = e & 3;
+    const int tr = pix / kHaloCols, tc = pix - tr * kHaloCols;
+    const int row = wrapi(h0 + tr - 1, H), col = wrapi(w0 + tc - 1, W);
+    src[i] = e < TP ? ((int64_t)(n * H + row) * W + col) * C + 8 * q : -1;
+  }
+  u32x4 rt[NTP], rw[NWP];
+  auto fetch_tile = [&](int c0) {
+#pragma unroll
+    for (int i = 0; i < NTP; ++i)
+      if (src[i] >= 0) rt[i] = *reinterpret_cast<const u32x4*>(x + src[i] + c0);
+  };
+  auto put_tile = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NTP; ++i) {
+      const int e = threadIdx.x + NT * i;
+      if (src[i] >= 0)
+        *reinterpret_cast<u32x4*>(tiles + b * kTile + (e >> 2) * kPixStride + 8 * (e & 3)) = rt[i];
+    }
+  };
+  // group g: taps 3*(g % 3) .. + 2 of chunk g / 3; piece e is lane e % 64's
+  // fragment of channel tile e / 64
+  auto fetch_w = [&](int g) {
+    const int tap0 = 3 * (g % 3), c0 = 32 * (g / 3);
+#pragma unroll
+    for (int i = 0; i < NWP; ++i) {
+      const int e = threadIdx.x + NT * i;
+      const int tap = e / (KB * 4), r = e % (KB * 4), l = r & 63;
+      if (WPC % NT == 0 || e < WPC)
+        rw[i] = *reinterpret_cast<const u32x4*>(
+            wt + ((int64_t)(tap0 + tap) * K + kb0 + (r >> 6) * 16 + (l & 15)) * C + c0 +
+            8 * (l >> 4));
+    }
+  };
+  auto put_w = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NWP; ++i) {
+      const int e = threadIdx.x + NT * i;
+      if (WPC % NT == 0 || e < WPC)
+        *reinterpret_cast<u32x4*>(weights + b * kW + 8 * e) = rw[i];
+    }
+  };
+
+  f32x4v acc[MW][NW];
+#pragma unroll
+  for (int m = 0; m < MW; ++m)
+#pragma unroll
+    for (int j = 0; j < NW; ++j) acc[m][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  const int nchunks = C / 32;
+  fetch_tile(0);
+  fetch_w(0);
+  put_tile(0);
+  put_w(0);
+  __syncthreads();
+  for (int ch = 0; ch < nchunks; ++ch) {
+    const uint16_t* tb = tiles + (ch & 1) * kTile;
+    const bool more = ch + 1 < nchunks;
+#pragma unroll
+    for (int dr = 0; dr < 3; ++dr) {
+      const int g = 3 * ch + dr;
+      if (dr < 2 || more) fetch_w(g + 1);
+      if (dr == 0 && more) fetch_tile(32 * (ch + 1));
+      const uint16_t* wb = weights + (g & 1) * kW + 8 * lane;
+#pragma unroll
+      for (int ds = 0; ds < 3; ++ds) {
+        bf16x8 a[MW], b[NW];
+#pragma unroll
+        for (int m = 0; m < MW; ++m)
+          a[m] = __builtin_bit_cast(
+              bf16x8, *reinterpret_cast<const u32x4*>(
+                          wb + ((ds * (KB / 16)) + wm * MW + m) * 512));
+#pragma unroll
+        for (int j = 0; j < NW; ++j)
+          b[j] = __builtin_bit_cast(
+              bf16x8, *reinterpret_cast<const u32x4*>(
+                          tb + ((wn * NW + j + dr) * kHaloCols + (lane & 15) + ds) * kPixStride +
+                          cq));
+#pragma unroll
+        for (int m = 0; m < MW; ++m)
+#pragma unroll
+          for (int j = 0; j < NW; ++j)
+            acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], b[j], acc[m][j], 0, 0, 0);
+      }
+      if (dr < 2 || more) put_w((g + 1) & 1);
+      if (dr == 2 && more) put_tile((ch + 1) & 1);
+      __syncthreads();
+    }
+  }
+
+  if constexpr (EPI == SPS_NN_EPI_PLAIN) {
+    store_plain<KB, TH * kTileCols, NT>(
+        acc, reinterpret_cast<uint16_t*>(lds), wn * NW * kTileCols + (lane & 15),
+        16 * MW * wm + 4 * (lane >> 4), bias ? bias + kb0 : nullptr, act, y, pre,
+        ((int64_t)(n * H + h0) * W + w0) * K + kb0, W, K);
+    return;
+  }
+  // upsample-add epilogue through LDS, half of the rows at a time: FP32 sums
+  // with the bias, then runs of pixels x channels in 16-byte pieces
+  float* stage = reinterpret_cast<float*>(lds);
+  constexpr int G = KB / 8;
+  for (int half = 0; half < 2; ++half) {
+    if (wn / (WN / 2) == half) {
+#pragma unroll
+      for (int m = 0; m < MW; ++m) {
+        const int cl = 16 * (MW * wm + m) + 4 * (lane >> 4);
+        float bv[4] = {0.f, 0.f, 0.f, 0.f};
+        if (bias) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) bv[i] = bias[kb0 + cl + i];
+        }
+#pragma unroll
+        for (int j = 0; j < NW; ++j) {
+          const int px = (wn % (WN / 2) * NW + j) * kTileCols + (lane & 15);
+          *reinterpret_cast<f32x4v*>(&stage[px * SKB + cl]) =
+              f32x4v{acc[m][j][0] + bv[0], acc[m][j][1] + bv[1], acc[m][j][2] + bv[2],
+                     acc[m][j][3] + bv[3]};
+        }
+      }
+    }
+    __syncthreads();
+    const int hb = h0 + half * (TH / 2);
+    {
+      constexpr int ITERS = 4 * PXH * G / NT, U = 4;
+      static_assert(ITERS % U == 0, "whole iterations");
+      for (int it = 0; it < ITERS; it += U) {
+        int64_t o[U];
+        int sp[U];
+        float u[U][8];
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+          const int e = threadIdx.x + NT * (it + q);
+          const int opx = e / G, g = e - opx * G;
+          const int orow = opx / (2 * kTileCols), ocol = opx % (2 * kTileCols);
+          sp[q] = ((orow >> 1) * kTileCols + (ocol >> 1)) * SKB + 8 * g;
+          o[q] = ((int64_t)(n * 2 * H + 2 * hb + orow) * (2 * W) + 2 * w0 + ocol) * K + kb0 +
+                 8 * g;
+          load8(skip + o[q], u[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < U; ++q) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) u[q][i] += stage[sp[q] + i];
+          if (pre) store8(pre + o[q], u[q]);
+          if (act) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) u[q][i] = silu(u[q][i]);
+          }
+          store8(y + o[q], u[q]);
+        }
+      }
+    }
+    __syncthreads();
   }
 }
 
@@ -1475,6 +1743,28 @@ int sps_nn_conv3x3(const void* x, int n, int h, int w, int cin,
   // 8 or 16 rows, 32 / 64 / 128 output channels per workgroup
   if (w % kTileCols == 0) {
     const int tiles_w = w / kTileCols;
+    // 8-wave tiles for two chunks of input channels and more (32->64 at 128^2,
+    // batch 64: 90 us, conv_fwd_tile 85), where they occupy half of the 256
+    // CUs at least (256->128 at 32^2 with the upsample-add epilogue,
+    // batch 32, 128 workgroups: 51 us, conv_fwd_tile 78)
+#define SPS_CONV_WIDE(WM, WN)                                                  \
+  do {                                                                         \
+    const int64_t wgs =                                                        \
+        h % (4 * (WN)) || cout % (64 * (WM))                                   \
+            ? 0                                                                \
+            : (int64_t)n * (h / (4 * (WN))) * tiles_w * (cout / (64 * (WM)));  \
+    if (cin == 32 || wgs < 128) break;                                         \
+    if (epilogue == SPS_NN_EPI_PLAIN)                                          \
+      conv_fwd_wide<WM, WN, 0><<<(unsigned)wgs, 512, 0, s>>>(                  \
+          xx, h, w, cin, ww, bias, cout, act, sk, yy, pp);                     \
+    else                                                                       \
+      conv_fwd_wide<WM, WN, 1><<<(unsigned)wgs, 512, 0, s>>>(                  \
+          xx, h, w, cin, ww, bias, cout, act, sk, yy, pp);                     \
+    return launch_ok("sps_nn_conv3x3");                                        \
+  } while (0)
+    SPS_CONV_WIDE(2, 4);
+    SPS_CONV_WIDE(1, 8);
+#undef SPS_CONV_WIDE
 #define SPS_CONV_TILE(MW, NW, WM, WN)                                           \
   do {                                                                         \
     constexpr int TH_ = (NW) * (WN), KB_ = 16 * (MW) * (WM);                   \
