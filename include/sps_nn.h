@@ -46,11 +46,9 @@ int sps_nn_conv3x3(const void* x, int n, int h, int w, int cin,
 
 /* Weight gradients are deterministic: each workgroup reduces its share of
  * the pixels in a fixed order into its own partial gradient in a caller-owned
- * FP32 workspace; a fixed tree then adds the partials to dweight (runs of
- * 32 partials summed in order, in place in the workspace, until at most 32
- * remain, which are added to dweight in order).  The same inputs give the
- * same bits on every call.  The workspace is scratch: its contents are
- * consumed.
+ * FP32 workspace; a fixed tree then adds the partials to dweight (16 or 4
+ * equal ranges of them, each summed in order, then the ranges in order).  The
+ * same inputs give the same bits on every call.  The workspace is scratch.
  * sps_nn_wgrad_workspace gives the workspace size in floats for a layer
  * (kind SPS_NN_WGRAD_CONV with cin and cout, SPS_NN_WGRAD_IN1 with cout,
  * SPS_NN_WGRAD_OUT1 with cin); 0 for invalid sizes. */
@@ -84,6 +82,13 @@ int sps_nn_conv3x3_in1(const float* x, int n, int h, int w,
 int sps_nn_conv3x3_in1_wgrad(const float* x, const void* dpre, int n, int h,
                              int w, int cout, float* dweight, float* workspace,
                              size_t ws_floats, void* stream);
+
+/* The same with the bias gradient, dbias[k] += sum dpre[p][k] (dbias NULL: the
+ * weight gradient alone). */
+int sps_nn_conv3x3_in1_wgrad_bias(const float* x, const void* dpre, int n,
+                                  int h, int w, int cout, float* dweight,
+                                  float* dbias, float* workspace,
+                                  size_t ws_floats, void* stream);
 
 /* Last layer, one FP32 output channel:
  *   y[n,h,w] = bias[0] + sum_{t,c} x[n, shift_t(h,w), c] * weight[t][c],

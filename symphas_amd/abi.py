@@ -198,6 +198,7 @@ def load() -> ctypes.CDLL:
         "sps_nn_wgrad_workspace": (c_size_t, [I, I, I, I, I, I]),
         "sps_nn_conv3x3_in1": (c_int, [P, I, I, I, P, P, I, I, P, P, P]),
         "sps_nn_conv3x3_in1_wgrad": (c_int, [P, P, I, I, I, I, P, P, c_size_t, P]),
+        "sps_nn_conv3x3_in1_wgrad_bias": (c_int, [P, P, I, I, I, I, P, P, P, c_size_t, P]),
         "sps_nn_conv3x3_out1": (c_int, [P, I, I, I, I, P, P, P, P]),
         "sps_nn_conv3x3_out1_bwd": (c_int, [P, P, I, I, I, I, P, P, P, P, c_size_t, P]),
         "sps_nn_silu_bwd": (c_int, [P, P, P, c_size_t, P]),

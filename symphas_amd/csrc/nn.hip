@@ -1192,57 +1192,72 @@ __global__ __launch_bounds__(256) void out1_fwd_tile(
   y[(int64_t)(n * H + h0 + ty) * W + w0 + tx] = v;
 }
 
-// dweight[t][k] += sum_p x[shift_t(p)] * dy[p][k]: 256-pixel chunks staged
-// in LDS, then thread (t, k) pairs reduce the chunk.
-__global__ __launch_bounds__(256) void in1_wgrad(const float* __restrict__ x,
-                                                 const uint16_t* __restrict__ dy,
-                                                 int N, int H, int W, int K,
-                                                 float* __restrict__ part,
-                                                 int chunks_per_block) {
-  __shared__ float sx[9][256];
-  __shared__ float sd[256][65];
-  const int64_t np = (int64_t)N * H * W;
+// Weight gradients of the thin layers: part[t][c] = sum_q a[q][c] * s[q'], q'
+// the pixel one tap away, (h + dr, w + ds) for SIGN = 1 (the first layer: a the
+// gradient, s the input) and (h - dr, w - ds) for SIGN = -1 (the last layer: a
+// the input, s the gradient); part[9][c] = sum_q a[q][c], the first layer's
+// bias gradient.  A lane is a pixel and keeps the 80 sums of 8 channels in
+// registers; a workgroup's 4 waves take neighbouring channels of the same
+// pixels, whose cache lines they share.  The lanes are added by halving (each
+// step a lane gives away half of its sums).  With a thread per (tap, channel)
+// and the pixels in LDS, two reads per product, the two layers took 100 and 115
+// us at 32 channels, 256^2, batch 32; this way 43 and 45.
+template <int SIGN>
+__global__ __launch_bounds__(256) void thin_wgrad(
+    const uint16_t* __restrict__ a, const float* __restrict__ s, int64_t np,
+    int H, int W, int C, float* __restrict__ part, int64_t slice, int64_t per,
+    int with_bias) {
+  const int lane = threadIdx.x & 63;
+  const int c0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * 8;
+  if (c0 >= C) return;
+  const int64_t p0 = blockIdx.x * per, p1 = min(np, p0 + per);
   const int HW = H * W;
-  float acc[3] = {0.f, 0.f, 0.f};  // up to 9*64 = 576 (t, k) pairs / 256
-  for (int c = 0; c < chunks_per_block; ++c) {
-    const int64_t base = ((int64_t)blockIdx.x * chunks_per_block + c) * 256;
-    if (base >= np) break;
-    __syncthreads();
-    const int64_t p = base + threadIdx.x;
-    if (p < np) {
-      const int n = p / HW, r = p - (int64_t)n * HW, h = r / W, w = r - h * W;
+  int64_t p = p0 + lane;
+  int64_t img = p / HW;
+  int h = (int)(p - img * HW) / W, w = (int)(p - img * HW) - h * W;
+  float v[80];
 #pragma unroll
-      for (int t = 0; t < 9; ++t)
-        sx[t][threadIdx.x] = x[(int64_t)(n * H + wrapi(h + t / 3 - 1, H)) * W +
-                               wrapi(w + t % 3 - 1, W)];
-      for (int k0 = 0; k0 < K; k0 += 8) {
-        float v[8];
-        load8(dy + p * K + k0, v);
+  for (int i = 0; i < 80; ++i) v[i] = 0.f;
+  for (; p < p1; p += 64) {
+    float x[8], sv[9];
+    load8(a + p * C + c0, x);
+    const float* si = s + img * HW;
+    const int hr[3] = {h == 0 ? H - 1 : h - 1, h, h + 1 == H ? 0 : h + 1};
+    const int wr[3] = {w == 0 ? W - 1 : w - 1, w, w + 1 == W ? 0 : w + 1};
 #pragma unroll
-        for (int i = 0; i < 8; ++i) sd[threadIdx.x][k0 + i] = v[i];
+    for (int t = 0; t < 9; ++t)
+      sv[t] = si[hr[SIGN > 0 ? t / 3 : 2 - t / 3] * W + wr[SIGN > 0 ? t % 3 : 2 - t % 3]];
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[8 * t + i] = fmaf(sv[t], x[i], v[8 * t + i]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[72 + i] += x[i];
+    for (w += 64; w >= W; w -= W)
+      if (++h == H) {
+        h = 0;
+        ++img;
       }
-    } else {
-#pragma unroll
-      for (int t = 0; t < 9; ++t) sx[t][threadIdx.x] = 0.f;
-      for (int k = 0; k < K; ++k) sd[threadIdx.x][k] = 0.f;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int tk = threadIdx.x + 256 * q;
-      if (tk < 9 * K) {
-        const int t = tk / K, k = tk - t * K;
-        float a = acc[q];
-        for (int i = 0; i < 256; ++i) a = fmaf(sx[t][i], sd[i][k], a);
-        acc[q] = a;
-      }
-    }
   }
-  float* dw = part + (int64_t)blockIdx.x * 9 * K;  // this block's partials
+  int first = 0;  // which of the 80 sums v[0] is
 #pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const int tk = threadIdx.x + 256 * q;
-    if (tk < 9 * K) dw[tk] = acc[q];
+  for (int st = 0; st < 4; ++st) {
+    const int n = 40 >> st, mask = 32 >> st;
+    const bool up = lane & mask;
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      const float give = up ? v[i] : v[n + i], keep = up ? v[n + i] : v[i];
+      v[i] = keep + __shfl_xor(give, mask, 64);
+    }
+    if (up) first += n;
+  }
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    v[i] += __shfl_xor(v[i], 2, 64);
+    v[i] += __shfl_xor(v[i], 1, 64);
+    const int t = (first + i) / 8, c = c0 + (first + i) % 8;
+    if ((lane & 3) == 0 && (t < 9 || with_bias))
+      part[blockIdx.x * slice + (int64_t)t * C + c] = v[i];
   }
 }
 
@@ -1296,146 +1311,37 @@ __global__ __launch_bounds__(256) void out1_bwd_data(
   }
 }
 
-// dweight[t][c] += sum_p x[shift_t(p)][c] * dy[p]: per 256-pixel chunk the
-// 9 shifted rows of x are read by thread (t, c) pairs from global memory
-// (L1/L2 hits) and dy from LDS.
-__global__ __launch_bounds__(256) void out1_wgrad(const uint16_t* __restrict__ x,
-                                                  const float* __restrict__ dy,
-                                                  int N, int H, int W, int C,
-                                                  float* __restrict__ part,
-                                                  int chunks_per_block) {
-  __shared__ float sd[256];
-  __shared__ int soff[9][256];
-  const int64_t np = (int64_t)N * H * W;
-  const int HW = H * W;
-  float acc[3] = {0.f, 0.f, 0.f};
-  for (int c = 0; c < chunks_per_block; ++c) {
-    const int64_t base = ((int64_t)blockIdx.x * chunks_per_block + c) * 256;
-    if (base >= np) break;
-    __syncthreads();
-    const int64_t p = base + threadIdx.x;
-    if (p < np) {
-      const int n = p / HW, r = p - (int64_t)n * HW, h = r / W, w = r - h * W;
-      sd[threadIdx.x] = dy[p];
+// The deterministic sum of M partial gradients of `count` floats each: a
+// workgroup takes 64 of the floats, its WAVES waves equal ranges of the partials
+// in order, and the ranges are added in order.  The first nw sums go to dw, the
+// others (a bias gradient) to db.  (Two launches, runs of 32 in place first,
+// took 11 + 6 us a layer; one 6.)
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void add_partials(
+    const float* __restrict__ part, int M, int64_t count, float* __restrict__ dw,
+    int64_t nw, float* __restrict__ db) {
+  __shared__ float sh[WAVES][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t i = (int64_t)blockIdx.x * 64 + lane;
+  const int m1 = (int)((int64_t)M * (wave + 1) / WAVES);
+  float s = 0.f;
+  if (i < count) {
+    int m = (int)((int64_t)M * wave / WAVES);
+    for (; m + 8 <= m1; m += 8) {
+      float v[8];
 #pragma unroll
-      for (int t = 0; t < 9; ++t)
-        soff[t][threadIdx.x] =
-            (int)((int64_t)(n * H + wrapi(h + t / 3 - 1, H)) * W +
-                  wrapi(w + t % 3 - 1, W) - base);
-    } else {
-      sd[threadIdx.x] = 0.f;
+      for (int q = 0; q < 8; ++q) v[q] = part[(int64_t)(m + q) * count + i];
 #pragma unroll
-      for (int t = 0; t < 9; ++t) soff[t][threadIdx.x] = 0;
+      for (int q = 0; q < 8; ++q) s += v[q];
     }
-    __syncthreads();
-    const int64_t lim = np - base;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int tc = threadIdx.x + 256 * q;
-      if (tc < 9 * C) {
-        const int t = tc / C, ch = tc - t * C;
-        float a = acc[q];
-        for (int i = 0; i < 256 && i < lim; ++i)
-          a = fmaf(bf2f(x[(base + soff[t][i]) * C + ch]), sd[i], a);
-        acc[q] = a;
-      }
-    }
+    for (; m < m1; ++m) s += part[(int64_t)m * count + i];
   }
-  float* dw = part + (int64_t)blockIdx.x * 9 * C;  // this block's partials
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const int tc = threadIdx.x + 256 * q;
-    if (tc < 9 * C) dw[tc] = acc[q];
-  }
-}
-
-// Weight gradient of the last layer on 16 x 16 pixel tiles: the x tile with
-// its periodic halo (18 x 18 pixels x C channels, BF16) and the tile's dy
-// (FP32) are staged in LDS, and thread (t, c) sums x[shift_t(p)][c] * dy[p]
-// over the tile's pixels in a fixed order.  A block walks tiles blockIdx.x,
-// + gridDim.x, ... and writes its partial sums to part[blockIdx.x][9][C].
-template <int C>
-__global__ __launch_bounds__(256) void out1_wgrad_tile(
-    const uint16_t* __restrict__ x, const float* __restrict__ dy, int N, int H,
-    int W, float* __restrict__ part) {
-  constexpr int T = 16, HT = T + 2, PS = C + 8, G = C / 8;
-  __shared__ __align__(16) uint16_t sx[HT * HT * PS];
-  __shared__ float sd[T * T];
-  const int tiles_w = W / T, tiles_h = H / T;
-  const int ntiles = N * tiles_h * tiles_w;
-  float acc[3] = {0.f, 0.f, 0.f};
-  for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    int b = tile;
-    const int tw = b % tiles_w;
-    b /= tiles_w;
-    const int th = b % tiles_h;
-    const int n = b / tiles_h;
-    const int h0 = th * T, w0 = tw * T;
-    __syncthreads();  // the previous tile's reads are done
-    for (int e = threadIdx.x; e < HT * HT * G; e += 256) {
-      const int pix = e / G, q = e - pix * G;
-      const int tr = pix / HT, tc = pix - tr * HT;
-      const int row = wrapi(h0 + tr - 1, H), col = wrapi(w0 + tc - 1, W);
-      *reinterpret_cast<u32x4*>(&sx[pix * PS + 8 * q]) =
-          *reinterpret_cast<const u32x4*>(x + ((int64_t)(n * H + row) * W + col) * C + 8 * q);
-    }
-    sd[threadIdx.x] =
-        dy[(int64_t)(n * H + h0 + threadIdx.x / T) * W + w0 + threadIdx.x % T];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int tc = threadIdx.x + 256 * q;
-      if (tc < 9 * C) {
-        const int t = tc / C, ch = tc - t * C;
-        const int dr = t / 3, ds = t % 3;
-        float a = acc[q];
-        for (int py = 0; py < T; ++py)
-#pragma unroll 4
-          for (int px = 0; px < T; ++px)
-            a = fmaf(bf2f(sx[((py + dr) * HT + px + ds) * PS + ch]), sd[py * T + px], a);
-        acc[q] = a;
-      }
-    }
-  }
-  float* dw = part + (int64_t)blockIdx.x * 9 * C;
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    const int tc = threadIdx.x + 256 * q;
-    if (tc < 9 * C) dw[tc] = acc[q];
-  }
-}
-
-// The deterministic sum of the per-block partial weight gradients, as a
-// fixed tree: the live partials sit in slots m*S of the workspace (m < M,
-// `count` floats per slot).  sum_partial_groups adds each run of gs of them,
-// in order, into the run's first slot (one thread per (run, weight), in
-// place); add_partials then adds the last M <= gs, in order, into dw.
-__global__ __launch_bounds__(256) void sum_partial_groups(float* __restrict__ part,
-                                                          int64_t count, int M,
-                                                          int64_t S, int gs) {
-  const int64_t ng = (M + gs - 1) / gs;
-  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < ng * count;
-       t += (int64_t)gridDim.x * 256) {
-    const int64_t g = t / count, i = t - g * count;
-    const int m0 = (int)g * gs, m1 = min(M, m0 + gs);
-    float s = 0.f;
-    for (int m = m0; m < m1; ++m) s += part[(int64_t)m * S * count + i];
-    part[(int64_t)m0 * S * count + i] = s;
-  }
-}
-
-// The first nw sums go to dw, the others (a bias gradient) to db.
-__global__ __launch_bounds__(256) void add_partials(const float* __restrict__ part,
-                                                    int M, int64_t S, int64_t count,
-                                                    float* __restrict__ dw, int64_t nw,
-                                                    float* __restrict__ db) {
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count;
-       i += (int64_t)gridDim.x * 256) {
-    float s = 0.f;
-    for (int m = 0; m < M; ++m) s += part[(int64_t)m * S * count + i];
-    if (i < nw) dw[i] += s;
-    else db[i - nw] += s;
-  }
+  sh[wave][lane] = s;
+  __syncthreads();
+  if (wave > 0 || i >= count) return;
+  for (int q = 1; q < WAVES; ++q) s += sh[q][lane];
+  if (i < nw) dw[i] += s;
+  else db[i - nw] += s;
 }
 
 // Bias gradient of the general path: workgroup z sums channels of its pixels.
@@ -1635,7 +1541,7 @@ constexpr int64_t kPartFloats = (int64_t)16 << 20;  // partial sums, at most
 
 struct WgradSplit {
   int blocks;    // workgroups that write a partial gradient
-  int per;       // chunks / tiles per workgroup
+  int per;       // chunks (thin layers: pixels) per workgroup
   int64_t count; // floats of one partial gradient
 };
 
@@ -1666,38 +1572,22 @@ WgradSplit conv_split(int n, int h, int w, int cin, int cout) {
   return {(int)((nchunks + per - 1) / per), (int)per, count};
 }
 
-WgradSplit chunk_split(int64_t np, int64_t count) {
-  const int64_t chunks = (np + 255) / 256;
-  const int64_t per = std::max<int64_t>(16, (chunks + 2047) / 2048);
-  return {(int)((chunks + per - 1) / per), (int)per, count};
+// The thin layers: at most 1024 workgroups (four waves per SIMD) of 16 runs of
+// 64 pixels at least, so that the partials stay a small share of what is read.
+WgradSplit thin_split(int64_t np, int64_t count) {
+  const int64_t runs = (np + 63) / 64;
+  const int64_t per = std::max<int64_t>(16, (runs + 1023) / 1024);
+  return {(int)((runs + per - 1) / per), (int)per * 64, count};
 }
 
-bool out1_tiled(int h, int w, int c) {
-  return h % 16 == 0 && w % 16 == 0 && (c == 32 || c == 64);
-}
-
-WgradSplit out1_split(int n, int h, int w, int c) {
-  if (!out1_tiled(h, w, c)) return chunk_split((int64_t)n * h * w, 9 * c);
-  const int64_t tiles = (int64_t)n * (h / 16) * (w / 16);
-  const int64_t per = (tiles + 2047) / 2048;
-  return {(int)((tiles + per - 1) / per), (int)per, (int64_t)9 * c};
-}
-
-// The workspace's partials are consumed (summed in place).
-int add_parts(float* part, const WgradSplit& sp, float* dw, hipStream_t s,
+int add_parts(const float* part, const WgradSplit& sp, float* dw, hipStream_t s,
               int64_t nw = -1, float* db = nullptr) {
-  constexpr int kGroup = 32;
-  int M = sp.blocks;
-  int64_t S = 1;
-  while (M > kGroup) {
-    const int64_t ng = (M + kGroup - 1) / kGroup;
-    sum_partial_groups<<<grid_for(ng * sp.count), 256, 0, s>>>(part, sp.count, M, S, kGroup);
-    SPS_TRY(launch_ok("weight-gradient partial sum"));
-    M = (int)ng;
-    S *= kGroup;
-  }
-  add_partials<<<grid_for(sp.count), 256, 0, s>>>(part, M, S, sp.count, dw,
-                                                  nw < 0 ? sp.count : nw, db);
+  if (nw < 0) nw = sp.count;
+  const unsigned blocks = (unsigned)((sp.count + 63) / 64);
+  if (sp.blocks > 32)
+    add_partials<16><<<blocks, 1024, 0, s>>>(part, sp.blocks, sp.count, dw, nw, db);
+  else
+    add_partials<4><<<blocks, 256, 0, s>>>(part, sp.blocks, sp.count, dw, nw, db);
   return launch_ok("weight-gradient partial sum");
 }
 
@@ -1822,8 +1712,8 @@ size_t sps_nn_wgrad_workspace(int kind, int n, int h, int w, int cin,
   if (kind == SPS_NN_WGRAD_CONV) {
     sp = conv_split(n, h, w, cin, cout);
     sp.count += cout;  // the bias gradient
-  } else if (kind == SPS_NN_WGRAD_IN1) sp = chunk_split(np, (int64_t)9 * cout);
-  else if (kind == SPS_NN_WGRAD_OUT1) sp = out1_split(n, h, w, cin);
+  } else if (kind == SPS_NN_WGRAD_IN1) sp = thin_split(np, (int64_t)10 * cout);
+  else if (kind == SPS_NN_WGRAD_OUT1) sp = thin_split(np, (int64_t)9 * cin);
   return (size_t)((int64_t)sp.blocks * sp.count);
 }
 
@@ -1920,18 +1810,27 @@ int sps_nn_conv3x3_in1(const float* x, int n, int h, int w,
 int sps_nn_conv3x3_in1_wgrad(const float* x, const void* dpre, int n, int h,
                              int w, int cout, float* dweight, float* workspace,
                              size_t ws_floats, void* stream) {
+  return sps_nn_conv3x3_in1_wgrad_bias(x, dpre, n, h, w, cout, dweight, nullptr,
+                                       workspace, ws_floats, stream);
+}
+
+int sps_nn_conv3x3_in1_wgrad_bias(const float* x, const void* dpre, int n,
+                                  int h, int w, int cout, float* dweight,
+                                  float* dbias, float* workspace,
+                                  size_t ws_floats, void* stream) {
   const int64_t np = (int64_t)n * h * w;
   if (!x || !dpre || !dweight || np < 1 || cout < 8 || cout > 64 || cout % 8) {
     set_error("sps_nn_conv3x3_in1_wgrad: cout a multiple of 8 in 8..64");
     return SPS_E_INVALID;
   }
-  const WgradSplit sp = chunk_split(np, (int64_t)9 * cout);
+  const WgradSplit sp = thin_split(np, (int64_t)(dbias ? 10 : 9) * cout);
   SPS_TRY(check_ws("sps_nn_conv3x3_in1_wgrad", sp, workspace, ws_floats));
   hipStream_t s = (hipStream_t)stream;
-  in1_wgrad<<<(unsigned)sp.blocks, 256, 0, s>>>(x, (const uint16_t*)dpre, n, h,
-                                                 w, cout, workspace, sp.per);
+  thin_wgrad<1><<<dim3((unsigned)sp.blocks, (cout + 31) / 32), 256, 0, s>>>(
+      (const uint16_t*)dpre, x, np, h, w, cout, workspace, sp.count, sp.per,
+      dbias != nullptr);
   SPS_TRY(launch_ok("sps_nn_conv3x3_in1_wgrad"));
-  return add_parts(workspace, sp, dweight, s);
+  return add_parts(workspace, sp, dweight, s, (int64_t)9 * cout, dbias);
 }
 
 int sps_nn_conv3x3_out1(const void* x, int n, int h, int w, int cin,
@@ -1965,7 +1864,7 @@ int sps_nn_conv3x3_out1_bwd(const void* x, const float* dy, int n, int h,
     return SPS_E_INVALID;
   }
   hipStream_t s = (hipStream_t)stream;
-  const WgradSplit sp = out1_split(n, h, w, cin);
+  const WgradSplit sp = thin_split(np, (int64_t)9 * cin);
   if (dweight) SPS_TRY(check_ws("sps_nn_conv3x3_out1_bwd", sp, workspace, ws_floats));
   if (dx) {
     out1_bwd_data<<<(unsigned)((np + 255) / 256), 256, 0, s>>>(
@@ -1973,14 +1872,8 @@ int sps_nn_conv3x3_out1_bwd(const void* x, const float* dy, int n, int h,
     SPS_TRY(launch_ok("sps_nn_conv3x3_out1_bwd (data)"));
   }
   if (dweight) {
-    const uint16_t* xx = (const uint16_t*)x;
-    if (out1_tiled(h, w, cin) && cin == 32)
-      out1_wgrad_tile<32><<<(unsigned)sp.blocks, 256, 0, s>>>(xx, dy, n, h, w, workspace);
-    else if (out1_tiled(h, w, cin))
-      out1_wgrad_tile<64><<<(unsigned)sp.blocks, 256, 0, s>>>(xx, dy, n, h, w, workspace);
-    else
-      out1_wgrad<<<(unsigned)sp.blocks, 256, 0, s>>>(xx, dy, n, h, w, cin, workspace,
-                                                      sp.per);
+    thin_wgrad<-1><<<dim3((unsigned)sp.blocks, (cin + 31) / 32), 256, 0, s>>>(
+        (const uint16_t*)x, dy, np, h, w, cin, workspace, sp.count, sp.per, 0);
     SPS_TRY(launch_ok("sps_nn_conv3x3_out1_bwd (weight)"));
     SPS_TRY(add_parts(workspace, sp, dweight, s));
   }

@@ -164,11 +164,12 @@ class _In1(torch.autograd.Function):
         dpre = silu_bwd_raw(dy, pre) if ctx.act == ACT_SILU else dy
         N, H, W = x.shape
         K = w.shape[1]
-        dw = torch.zeros((9, K), device=x.device, dtype=torch.float32)
+        g = torch.zeros((10, K), device=x.device, dtype=torch.float32)
+        dw, db = g[:9], g[9]
         ws = wgrad_workspace(WGRAD_IN1, N, H, W, 1, K, x.device)
-        _check(_lib().sps_nn_conv3x3_in1_wgrad(_ptr(x.contiguous()), _ptr(dpre), N, H, W, K,
-                                               _ptr(dw), _ptr(ws), ws.numel(), _stream()))
-        db = torch.sum(dpre, dim=(0, 1, 2), dtype=torch.float32)
+        _check(_lib().sps_nn_conv3x3_in1_wgrad_bias(_ptr(x.contiguous()), _ptr(dpre), N, H, W, K,
+                                                    _ptr(dw), _ptr(db), _ptr(ws), ws.numel(),
+                                                    _stream()))
         return None, dw, db, None
 
 

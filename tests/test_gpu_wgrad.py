@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from symphas_amd import nn
+from symphas_amd import abi, nn
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +37,36 @@ def test_weight_and_bias_gradients(gpu_lib, N, H, W, C, K):
         assert float((dw[t].double() - want).abs().max()) <= tol * scale, t
     scale = float(dd.abs().sum(0).max()) / np.sqrt(N * H * W)
     assert float((db.double() - dd.sum(0)).abs().max()) <= tol * scale
+
+
+# one run of 64 pixels, a part of one, rows shorter than a run, several and
+# more than 1024 workgroups' least; channels that leave waves idle
+@pytest.mark.parametrize("N,H,W,C", [(1, 8, 8, 32), (1, 5, 7, 8), (3, 3, 3, 16), (2, 9, 70, 24),
+                                     (1, 1, 2000, 64), (5, 128, 128, 32), (2, 200, 331, 40),
+                                     (3, 700, 601, 8)])
+def test_thin_gradients(gpu_lib, N, H, W, C):
+    print("[case] thin wgrad", N, H, W, C, flush=True)
+    lib = abi.load()
+    g = torch.Generator(device="cuda").manual_seed(W)
+    a = torch.randn(N, H, W, C, device="cuda", generator=g).to(torch.bfloat16)
+    s = torch.randn(N, H, W, device="cuda", generator=g)
+    tol = 8 * 2.0 ** -24 * np.sqrt(N * H * W) + 2.0 ** -22
+    for kind, sign in ((nn.WGRAD_IN1, 1), (nn.WGRAD_OUT1, -1)):
+        out = torch.zeros(10, C, device="cuda")
+        ws = nn.wgrad_workspace(kind, N, H, W, C, C, "cuda")
+        if sign > 0:
+            nn._check(lib.sps_nn_conv3x3_in1_wgrad_bias(
+                nn._ptr(s), nn._ptr(a), N, H, W, C, nn._ptr(out), nn._ptr(out[9]), nn._ptr(ws),
+                ws.numel(), nn._stream()))
+            assert torch.allclose(out[9].double(), a.double().sum((0, 1, 2)), rtol=0,
+                                  atol=tol * np.sqrt(N * H * W))
+        else:
+            w = torch.zeros(9, C, device="cuda")
+            nn._check(lib.sps_nn_conv3x3_out1_bwd(
+                nn._ptr(a), nn._ptr(s), N, H, W, C, nn._ptr(w), None, nn._ptr(out), nn._ptr(ws),
+                ws.numel(), nn._stream()))
+        for t in range(9):
+            v = torch.roll(s, (sign * (1 - t // 3), sign * (1 - t % 3)), dims=(1, 2)).double()
+            want = (v[..., None] * a.double()).sum((0, 1, 2))
+            # sums of N*H*W unit products
+            assert float((out[t].double() - want).abs().max()) <= tol * np.sqrt(N * H * W), (kind, t)
