@@ -31,6 +31,7 @@
 #include "lanes.hpp"
 #include "plan.hpp"
 #include "ref_kernels.hpp"
+#include "shape.hpp"
 
 namespace sps {
 namespace {
@@ -430,22 +431,36 @@ __global__ __launch_bounds__(64) void box_stream2d(const T* __restrict__ in,
                                                        store_lane, c, bm);
 }
 
-// Chunk height of the box stream: about two waves per SIMD, at least 16 rows
-// (shorter chunks spend most of their rows on the pipeline fill).
-inline int box_stream_rows(int by, int nstrips, int cus) {
-  const int64_t target = 8LL * cus;  // waves
-  const int64_t nch = std::max<int64_t>(1, target / std::max(1, nstrips));
-  return (int)std::max<int64_t>(16, (by + nch - 1) / nch);
+// Chunk height of the box stream: the least of shape.hpp's cost over a few
+// heights (evaluated at every launch).  A wave computes its rows and the fill
+// of 2 x kBoxSteps x radius rows, so short chunks repeat more work, but the
+// launch is a chain of rows per wave and a box leaves SIMDs idle: at 16 rows
+// and more a box of 804^2 was 408 waves, at 7 rows it is 920.  2000 FP32 steps
+// of a 600^2 droplet in 2048^2 with its searches: 7.05 -> 5.75 ms.
+inline int box_stream_rows(int by, int nstrips, int fill) {
+  int best = 4;
+  double least = 0;
+  for (int rows : {4, 5, 6, 7, 8, 10, 12, 14, 16, 20, 24, 28, 32, 40, 48, 64, 96, 128, 256,
+                   512, 1024}) {
+    const int64_t waves = (int64_t)nstrips * ((by + rows - 1) / rows);
+    const double cost =
+        (rows + fill) * std::max(1.5, (double)((waves + kSimds - 1) / kSimds));
+    if (least == 0 || cost < least) {
+      least = cost;
+      best = rows;
+    }
+  }
+  return best;
 }
 
 template <typename T, int VEC, int R, bool HASA, int POLY>
 int launch_box_stream(const T* psi, T* out, const BoxGeom& g, const FusedCoef<T>& c,
-                      int cus, hipStream_t s) {
+                      hipStream_t s) {
   constexpr int HL = (kBoxSteps * R + VEC - 1) / VEC;
   constexpr int W = (64 - 2 * HL) * VEC;
   const int bx = g.b[0], by = g.b[1];
   const int nstrips = (bx + W - 1) / W;
-  const int TY = box_stream_rows(by, nstrips, cus);
+  const int TY = box_stream_rows(by, nstrips, 2 * kBoxSteps * R);
   const int nitems = nstrips * ((by + TY - 1) / TY);
   box_stream2d<T, VEC, R, HASA, POLY><<<nitems, 64, 0, s>>>(psi, out, bx, by, TY, nstrips,
                                                            nitems, c);
@@ -456,10 +471,10 @@ int launch_box_stream(const T* psi, T* out, const BoxGeom& g, const FusedCoef<T>
 // two values per lane (8-byte aligned rows), the others one.
 template <typename T>
 int box_multi_step(const T* psi, T* out, const BoxGeom& g, const FusedCoef<T>& c,
-                   int cus, hipStream_t s) {
+                   hipStream_t s) {
   const bool hasa = c.dega >= 0;
   const bool two = sizeof(T) == 4 && g.b[0] % 2 == 0;
-#define SPS_BOXS(V_, R_, A_, P_) launch_box_stream<T, V_, R_, A_, P_>(psi, out, g, c, cus, s)
+#define SPS_BOXS(V_, R_, A_, P_) launch_box_stream<T, V_, R_, A_, P_>(psi, out, g, c, s)
 #define SPS_BOXR(V_)                                                                   \
   (c.radius == 1                                                                       \
        ? (c.poly == 3 ? (hasa ? SPS_BOXS(V_, 1, true, 3) : SPS_BOXS(V_, 1, false, 3))  \
@@ -535,7 +550,6 @@ struct sps_fdr_plan {
   int o[3] = {0, 0, 0}, b[3] = {1, 1, 1};
   bool has_data = false, has_box = true;
   int next_resize = 0, index = 0;
-  int cus = 256;  // compute units of the plan's device (box stream chunking)
   double empty = 0.0, cutoff = 0.0, time = 0.0;
 
   sps::BoxGeom geom() const {
@@ -788,9 +802,9 @@ struct sps_fdr_plan {
         const int rc =
             d.dtype == SPS_F32
                 ? sps::box_multi_step<float>((const float*)box[cur], (float*)box[nxt], g,
-                                             fc32, cus, stream)
+                                             fc32, stream)
                 : sps::box_multi_step<double>((const double*)box[cur], (double*)box[nxt],
-                                              g, fc64, cus, stream);
+                                              g, fc64, stream);
         if (rc != SPS_OK) return rc;
         cur = nxt;
         for (int j = 0; j < sps::kBoxSteps; ++j) {
@@ -908,16 +922,6 @@ int sps_fdr_create(const sps_fd_desc* desc, const sps_fd_regional* params,
     p->stream = nullptr;
     set_error("hipStreamCreate failed: %s", hipGetErrorString(se));
     rc = SPS_E_HIP;
-  }
-  if (rc == SPS_OK) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&p->cus, hipDeviceAttributeMultiprocessorCount, dev) !=
-            hipSuccess ||
-        p->cus < 1) {
-      set_error("device query failed");
-      rc = SPS_E_HIP;
-    }
   }
   alloc(&p->box[0], p->cap * p->esize);
   alloc(&p->box[1], p->cap * p->esize);

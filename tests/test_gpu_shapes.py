@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 
 from symphas_amd import abi, inputs, models
-from symphas_amd.solver import FDBatch, FDPlan, MultiPlan
+from symphas_amd.solver import FDBatch, FDPlan, MultiPlan, RegionalPlan, interior_shape
 
 pytestmark = pytest.mark.gpu
 
@@ -111,3 +111,22 @@ def test_row_sums(gpu_lib, n, gradient, dtype):
     tol = (g.size + 16) * 2.0 ** -52
     assert abs(mass - g.sum()) <= tol * np.abs(g).sum()
     assert abs(energy - e.sum()) <= tol * np.abs(e).sum() * 4
+
+
+@pytest.mark.parametrize("dtype", [abi.F32, abi.F64])
+@pytest.mark.parametrize("blob", [(820, 790), (1210, 1300), (1700, 61)])
+def test_regional_box_chunks(gpu_lib, blob, dtype):
+    """Boxes whose chunk height is above the least one (7, 14 and more rows; a
+    short last chunk): four steps per launch against one, bit for bit."""
+    d = models.model_b((2048, 1600), dt=0.01, dtype=dtype, path=abi.PATH_FUSED)
+    psi = np.zeros(interior_shape(d), np.float32 if dtype == abi.F32 else np.float64)
+    psi[60:60 + blob[1], 50:50 + blob[0]] = 0.4 + field(blob, 31, dtype) * 0.05
+    got = {}
+    for spl in (1, 4):
+        with RegionalPlan(d, abi.Regional(1e-6, 1.1, 1.0, 1, spl, 0.05)) as rp:
+            rp.upload(psi)
+            rp.step(23)
+            info = rp.region()
+            assert blob[0] <= info.dims[0] < d.n[0] and blob[1] <= info.dims[1] < d.n[1]
+            got[spl] = rp.download()
+    assert np.array_equal(got[1], got[4])
