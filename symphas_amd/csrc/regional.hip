@@ -436,7 +436,7 @@ __global__ __launch_bounds__(64) void box_stream2d(const T* __restrict__ in,
 // of 2 x kBoxSteps x radius rows, so short chunks repeat more work, but the
 // launch is a chain of rows per wave and a box leaves SIMDs idle: at 16 rows
 // and more a box of 804^2 was 408 waves, at 7 rows it is 920.  2000 FP32 steps
-// of a 600^2 droplet in 2048^2 with its searches: 7.05 -> 5.75 ms.
+// of a droplet of radius 200 in 2048^2 with its searches: 7.05 -> 5.75 ms.
 inline int box_stream_rows(int by, int nstrips, int fill) {
   int best = 4;
   double least = 0;
