@@ -66,25 +66,29 @@ struct Stream3DCand {
   int steps, rows;
   double t;
 };
+// us per step
+inline double stream_cost3d(int X, int Y, int Z, int R, int esize, int fields,
+                            const Stream3DCand& c, int planes, double q) {
+  const double bytes = 1.0 * X * Y * Z * esize * fields;
+  const double hbm = 2 * bytes > 256e6 ? 2.3 * bytes / 5.3e6 : 0.0;
+  const int64_t strip = 64 - 2 * R * c.steps;
+  const int64_t waves = ((X + strip - 1) / strip) * ((Y + c.rows - 1) / c.rows) *
+                        ((Z + planes - 1) / planes);
+  const double w = (double)((waves + kSimds - 1) / kSimds);
+  const double run = (planes + 2 * R * c.steps) * std::max(q, w) * c.t;
+  return (3.2 + std::max(run, hbm)) / c.steps;
+}
 inline StreamShape stream_shape3d(int X, int Y, int Z, int R, int esize,
                                   int fields, const Stream3DCand* cand,
                                   int ncand, double q) {
-  const double bytes = 1.0 * X * Y * Z * esize * fields;
-  const double hbm = 2 * bytes > 256e6 ? 2.3 * bytes / 5.3e6 : 0.0;
   StreamShape best{1, cand[0].rows, 16, 1};
   double least = 0;
   for (int i = 0; i < ncand; ++i) {
-    const int k = cand[i].steps, rows = cand[i].rows;
-    const int64_t strip = 64 - 2 * R * k;
-    const int64_t per_chunk = ((X + strip - 1) / strip) * ((Y + rows - 1) / rows);
     for (int tz = 1; tz <= 1024; ++tz) {
-      const int64_t waves = per_chunk * ((Z + tz - 1) / tz);
-      const double w = (double)((waves + kSimds - 1) / kSimds);
-      const double run = (tz + 2 * R * k) * std::max(q, w) * cand[i].t;
-      const double cost = (3.2 + std::max(run, hbm)) / k;
+      const double cost = stream_cost3d(X, Y, Z, R, esize, fields, cand[i], tz, q);
       if (least == 0 || cost < least) {
         least = cost;
-        best = StreamShape{k, rows, tz, 1};
+        best = StreamShape{cand[i].steps, cand[i].rows, tz, 1};
       }
       if (tz >= Z) break;
     }

@@ -37,7 +37,8 @@ def test_default_shape_2d(gpu_lib, n, dtype):
 
 
 @pytest.mark.parametrize("dtype", [abi.F32, abi.F64])
-@pytest.mark.parametrize("n", [(3, 4, 5), (65, 13, 3), (60, 61, 62), (200, 70, 90)])
+@pytest.mark.parametrize("n", [(3, 4, 5), (65, 13, 3), (60, 61, 62), (200, 70, 90),
+                               (236, 232, 240), (300, 280, 250)])
 def test_default_shape_3d(gpu_lib, n, dtype):
     for model, kw in ((models.model_b, {"dt": 0.005}), (models.allen_cahn, {})):
         d = model(n, dtype=dtype, stencil=models.Stencil3d2h(7, 10, 25), **kw)
