@@ -212,25 +212,35 @@ def _file_bytes(call) -> bytes:
     """The bytes of a file: call(buffer, capacity, length) as the C entry points
     take them, asked for the length first and then to fill a bytes object of
     that length in place (filling a larger array and copying it out touches
-    fresh memory twice).  Large objects ask for huge pages first, as numpy's
-    arrays do: the copy from the device into 4 KiB pages that do not exist yet
-    spends most of its time on their faults (73 MB: 17.5 ms, huge pages 7.5).
-    Checkpoint text of 2048^2 FP32 values, in all: 26 ms that way, 8.7 this way."""
+    fresh memory twice).  Where the field was advanced between the two calls
+    the second text has a length of its own: a shorter one is cut to it, for a
+    longer one the call is made again.  Large objects ask for huge pages first,
+    as numpy's arrays do: the copy from the device into 4 KiB pages that do not
+    exist yet spends most of its time on their faults (73 MB: 17.5 ms, huge
+    pages 7.5).  Checkpoint text of 2048^2 FP32 values, in all: 26 ms that way,
+    8.7 this way."""
     n = c_size_t(0)
     abi.check(call(None, 0, byref(n)))
     api = ctypes.pythonapi
     new = ctypes.PYFUNCTYPE(ctypes.py_object, c_void_p, ctypes.c_ssize_t)(
         ("PyBytes_FromStringAndSize", api))
-    out = new(None, n.value)
-    at = ctypes.PYFUNCTYPE(c_void_p, ctypes.py_object)(("PyBytes_AsString", api))(out)
-    if n.value >= 1 << 22 and sys.platform == "linux":
-        page = mmap.PAGESIZE
-        first, end = -(-at // page) * page, (at + n.value) // page * page
-        madvise = ctypes.CDLL(None).madvise  # advice only: its result does not matter
-        madvise.argtypes = [c_void_p, c_size_t, c_int]
-        madvise(first, end - first, _MADV_HUGEPAGE)
-    abi.check(call(c_void_p(at), n.value, byref(n)))
-    return out
+    address = ctypes.PYFUNCTYPE(c_void_p, ctypes.py_object)(("PyBytes_AsString", api))
+    while True:
+        size = n.value
+        out = new(None, size)
+        at = address(out)
+        if size >= 1 << 22 and sys.platform == "linux":
+            page = mmap.PAGESIZE
+            first, end = -(-at // page) * page, (at + size) // page * page
+            madvise = ctypes.CDLL(None).madvise  # advice only: its result does not matter
+            madvise.argtypes = [c_void_p, c_size_t, c_int]
+            madvise(first, end - first, _MADV_HUGEPAGE)
+        rc = call(c_void_p(at), size, byref(n))
+        if rc == abi.OK and n.value <= size:
+            return out if n.value == size else out[:n.value]
+        abi.check(call(None, 0, byref(n)))
+        if n.value <= size:  # not for want of room
+            abi.check(rc)
 
 
 def checkpoint_progress(directory: str):
