@@ -6,7 +6,7 @@
 // (reduce_rows.hpp).  Waves reduce with xor shuffles, the waves of a block
 // through LDS.  Pass 2: one workgroup adds the partials in a fixed order and
 // applies the functional's scale (h^D, or 1/sites for the mean).  The result
-// is deterministic for a given field, size and alignment.
+// is deterministic for a given field and size, wherever the field lies.
 #include <mutex>
 
 #include "fused.hpp"
@@ -17,7 +17,7 @@ namespace {
 
 constexpr int kPass1Threads = 512;
 
-template <typename T, int VEC>
+template <typename T, int VEC, bool ALIGNED>
 __global__ __launch_bounds__(kPass1Threads) void reduce_pass1(
     const T* __restrict__ f, int dim, int X, int Y, int Z, EnergyParams ep,
     double* partials) {
@@ -27,7 +27,7 @@ __global__ __launch_bounds__(kPass1Threads) void reduce_pass1(
   const int r0 = (int)(rows * b / gridDim.x);
   const int r1 = (int)(rows * (b + 1) / gridDim.x);
   double m = 0.0, e = 0.0;
-  reduce_rows<T, VEC>(f, dim, X, Y, Z, r0, r1, ep, m, e);
+  reduce_rows<T, VEC, ALIGNED>(f, dim, X, Y, Z, r0, r1, ep, m, e);
   block_sum2<kPass1Threads / 64>(m, e);
   if (threadIdx.x == 0) {
     partials[2 * b] = m;
@@ -59,12 +59,15 @@ int launch_reduce(const T* f, int dim, const int* n, double h,
   const int X = n[0], Y = n[1], Z = dim == 3 ? n[2] : 1;
   const int rows = Y * Z;
   const int nb = rows < kReduceBlocks ? rows : kReduceBlocks;
-  // 16-byte groups where the rows and the field's address allow it
+  // groups of 16 bytes where they divide the rows, in one load each where the
+  // field's address allows it (a caller's may lie anywhere)
   constexpr int kVec = 16 / sizeof(T);
-  if (X % kVec == 0 && (uintptr_t)f % 16 == 0)
-    reduce_pass1<T, kVec><<<nb, kPass1Threads, 0, s>>>(f, dim, X, Y, Z, ep, partials);
+  if (X % kVec != 0)
+    reduce_pass1<T, 1, true><<<nb, kPass1Threads, 0, s>>>(f, dim, X, Y, Z, ep, partials);
+  else if ((uintptr_t)f % 16 == 0)
+    reduce_pass1<T, kVec, true><<<nb, kPass1Threads, 0, s>>>(f, dim, X, Y, Z, ep, partials);
   else
-    reduce_pass1<T, 1><<<nb, kPass1Threads, 0, s>>>(f, dim, X, Y, Z, ep, partials);
+    reduce_pass1<T, kVec, false><<<nb, kPass1Threads, 0, s>>>(f, dim, X, Y, Z, ep, partials);
   const double sites = (double)X * Y * Z;
   reduce_pass2<<<1, 256, 0, s>>>(partials, nb, energy_scale(ep, dim, h, sites),
                                  sums);

@@ -11,9 +11,10 @@ namespace sps {
 // takes VEC consecutive sites at a time: their values and the rows above come
 // as one load each, and the one x neighbour that is not among them as another.
 // With a scalar load per value and neighbour the sums of 512^3 FP32 took 0.58
-// ms (0.9 TB/s), on latency; this way 0.18 ms.  X must be a multiple of VEC and f aligned to
-// VEC values; Z = 1 in 2D.
-template <typename T, int VEC>
+// ms (0.9 TB/s), on latency; this way 0.18 ms.  X must be a multiple of VEC and
+// f aligned to VEC values, or ALIGNED false: the same groups, and so the same
+// order of the sums, loaded value by value.  Z = 1 in 2D.
+template <typename T, int VEC, bool ALIGNED = true>
 __device__ __forceinline__ void reduce_rows(const T* __restrict__ f, int dim,
                                             int X, int Y, int Z, int r0, int r1,
                                             const EnergyParams& ep, double& m,
@@ -27,18 +28,26 @@ __device__ __forceinline__ void reduce_rows(const T* __restrict__ f, int dim,
   int y = r % Y, z = r / Y;
   const bool central = ep.central != 0;
   const int64_t XY = (int64_t)X * Y;
+  auto load = [](const T* p, T (&v)[VEC]) {
+    if constexpr (ALIGNED) {
+      load_vec<VEC>(p, v);
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) v[j] = p[j];
+    }
+  };
   while (r < r1) {
     const int x = xg * VEC;
     const T* row = f + (int64_t)r * X;
     T v[VEC], up[VEC], dn[VEC];
-    load_vec<VEC>(row + x, v);
-    load_vec<VEC>((y + 1 == Y ? row - (XY - X) : row + X) + x, up);
+    load(row + x, v);
+    load((y + 1 == Y ? row - (XY - X) : row + X) + x, up);
     const T right = row[x + VEC == X ? 0 : x + VEC];
     T left = v[0];
     double g2[VEC];
     if (central) {
       left = row[x == 0 ? X - 1 : x - 1];
-      load_vec<VEC>((y == 0 ? row + (XY - X) : row - X) + x, dn);
+      load((y == 0 ? row + (XY - X) : row - X) + x, dn);
     }
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
@@ -49,8 +58,8 @@ __device__ __forceinline__ void reduce_rows(const T* __restrict__ f, int dim,
       g2[j] = gx * gx + gy * gy;
     }
     if (dim == 3) {
-      load_vec<VEC>((z + 1 == Z ? f + (int64_t)y * X : row + XY) + x, up);
-      if (central) load_vec<VEC>((z == 0 ? row + (Z - 1) * XY : row - XY) + x, dn);
+      load((z + 1 == Z ? f + (int64_t)y * X : row + XY) + x, up);
+      if (central) load((z == 0 ? row + (Z - 1) * XY : row - XY) + x, dn);
 #pragma unroll
       for (int j = 0; j < VEC; ++j) {
         const double gz = (double)up[j] - (double)(central ? dn[j] : v[j]);

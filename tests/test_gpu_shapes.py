@@ -131,3 +131,33 @@ def test_regional_box_chunks(gpu_lib, blob, dtype):
             assert blob[0] <= info.dims[0] < d.n[0] and blob[1] <= info.dims[1] < d.n[1]
             got[spl] = rp.download()
     assert np.array_equal(got[1], got[4])
+
+
+@pytest.mark.parametrize("dtype", [abi.F32, abi.F64])
+@pytest.mark.parametrize("n", [(64, 48), (260, 31), (36, 10, 9)])
+def test_sums_wherever_the_field_lies(gpu_lib, n, dtype):
+    # a caller's field may start at any value of an allocation: the sums are
+    # those of the plan bit for bit, in the order that the sizes alone set
+    import ctypes
+
+    import torch
+    st = {"stencil": models.Stencil3d2h(7, 10, 25), "dt": 0.005} if len(n) == 3 else {}
+    d = models.model_b(n, dtype=dtype, **st)
+    psi = field(n, 57, dtype)
+    energy = abi.Energy(0.7, 1.3, 1.9, abi.GRAD_CENTRAL, 0)
+    with FDPlan(d) as p:
+        p.upload(psi)
+        p.set_energy(energy)
+        want = p.reduce()
+    sums = torch.empty(2, device="cuda", dtype=torch.float64)
+    for shift in (0, 1, 3):
+        buf = torch.zeros(psi.size + 8, device="cuda",
+                          dtype=torch.float32 if dtype == abi.F32 else torch.float64)
+        buf[shift:shift + psi.size] = torch.from_numpy(psi.ravel()).to("cuda")
+        nn = (ctypes.c_int32 * 3)(*(list(n) + [1] * (3 - len(n))))
+        torch.cuda.synchronize()
+        abi.check(gpu_lib.sps_fd_reduce_device(
+            d.dim, dtype, nn, d.h, ctypes.byref(energy),
+            ctypes.c_void_p(buf[shift:].data_ptr()), ctypes.c_void_p(sums.data_ptr()), None))
+        torch.cuda.synchronize()
+        assert tuple(sums.cpu().tolist()) == want, shift
