@@ -743,6 +743,11 @@ __device__ __forceinline__ uint2 read_tr(const uint16_t* p) {
                  (__attribute__((address_space(3))) i16x4*)p));
 }
 
+__device__ __forceinline__ bf16x8 bf16_ones() {
+  constexpr uint32_t kOnes = 0x3f803f80u;  // two BF16 ones
+  return __builtin_bit_cast(bf16x8, u32x4{kOnes, kOnes, kOnes, kOnes});
+}
+
 template <int KT, int CT, int WC>
 struct WgradTile {
   static constexpr int kThreads = 512;
@@ -823,8 +828,6 @@ __global__ __launch_bounds__(512) void conv_wgrad_tile(
       for (int b = 0; b < 2; ++b) acc[t][a][b] = f32x4v{0.f, 0.f, 0.f, 0.f};
   accb[0] = accb[1] = f32x4v{0.f, 0.f, 0.f, 0.f};
   const bool bias_wave = with_bias && blockIdx.x == 0 && wc == 0;
-  constexpr uint32_t kOnes = 0x3f803f80u;  // two BF16 ones
-  const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{kOnes, kOnes, kOnes, kOnes});
 
   const int first = blockIdx.z * per, last = min(nchunks, first + per);
   if (first < last) {
@@ -851,7 +854,7 @@ __global__ __launch_bounds__(512) void conv_wgrad_tile(
       if (bias_wave) {
 #pragma unroll
         for (int tk = 0; tk < 2; ++tk)
-          accb[tk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tk], ones, accb[tk], 0, 0, 0);
+          accb[tk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tk], bf16_ones(), accb[tk], 0, 0, 0);
       }
 #pragma unroll
       for (int r = 0; r < 3; ++r)
@@ -938,11 +941,15 @@ __global__ __launch_bounds__(512) void conv_wgrad_tile(
 // ROWS: chunks are 32-pixel pieces of one row (w % 32 == 0) and the three
 // input rows with a 1-column halo are staged once; otherwise chunks are any
 // 32 consecutive pixels and the nine shifted pixels are staged per tap.
+// The bias gradient is a product of the staged dpre with ones, in two waves of
+// the first column of workgroups.  Layers of 256 channels, 56 images of 24^2
+// and 20 of 40^2, both gradients: 195 and 184 us; with a library sum of dpre
+// 227 and 216, with a kernel of one thread per channel 473 and 461.
 template <int KT, int CT, bool ROWS>
 __global__ __launch_bounds__(256) void conv_wgrad(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ dy, int N,
     int H, int W, int C, int K, float* __restrict__ part, int64_t slice,
-    int nchunks, int chunks_per_block) {
+    int nchunks, int chunks_per_block, int with_bias) {
   constexpr int TK = KT / 32, TC = CT / 32;  // MFMA tiles per wave
   __shared__ __align__(16) uint16_t sdy[32][KT + 2];
   __shared__ __align__(16) uint16_t sx[ROWS ? 3 : 9][ROWS ? 34 : 32][CT + 2];
@@ -957,6 +964,10 @@ __global__ __launch_bounds__(256) void conv_wgrad(
     for (int a = 0; a < TK; ++a)
 #pragma unroll
       for (int b = 0; b < TC; ++b) acc[t][a][b] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  f32x4v accb[TK];
+#pragma unroll
+  for (int a = 0; a < TK; ++a) accb[a] = f32x4v{0.f, 0.f, 0.f, 0.f};
+  const bool bias_wave = with_bias && blockIdx.x == 0 && wave < 2;
 
   const int first = blockIdx.z * chunks_per_block;
   const int last = min(nchunks, first + chunks_per_block);
@@ -1019,6 +1030,11 @@ __global__ __launch_bounds__(256) void conv_wgrad(
       for (int i = 0; i < 8; ++i) v[i] = sdy[pq + i][kw + 16 * tk + (lane & 15)];
       a[tk] = __builtin_bit_cast(bf16x8, v);
     }
+    if (bias_wave) {
+#pragma unroll
+      for (int tk = 0; tk < TK; ++tk)
+        accb[tk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tk], bf16_ones(), accb[tk], 0, 0, 0);
+    }
 #pragma unroll
     for (int tap = 0; tap < 9; ++tap) {
       const int r = tap / 3, s = tap % 3;
@@ -1054,6 +1070,13 @@ __global__ __launch_bounds__(256) void conv_wgrad(
           const int c = c0 + cw + 16 * tc + (lane & 15);
           dw[((int64_t)tap * K + k) * C + c] = acc[tap][tk][tc][i];
         }
+  if (bias_wave && (lane & 15) == 0) {
+#pragma unroll
+    for (int tk = 0; tk < TK; ++tk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        dw[(int64_t)9 * K * C + k0 + kw + 16 * tk + 4 * (lane >> 4) + i] = accb[tk][i];
+  }
 }
 
 // ------------------------------------------------------------ thin layers
@@ -1342,19 +1365,6 @@ __global__ __launch_bounds__(64 * WAVES) void add_partials(
   for (int q = 1; q < WAVES; ++q) s += sh[q][lane];
   if (i < nw) dw[i] += s;
   else db[i - nw] += s;
-}
-
-// Bias gradient of the general path: workgroup z sums channels of its pixels.
-__global__ __launch_bounds__(256) void bias_partials(const uint16_t* __restrict__ dy,
-                                                     int64_t npix, int K, int64_t per,
-                                                     float* __restrict__ part,
-                                                     int64_t slice) {
-  const int64_t p0 = blockIdx.x * per, p1 = min(npix, p0 + per);
-  for (int k = threadIdx.x; k < K; k += 256) {
-    float s = 0.f;
-    for (int64_t p = p0; p < p1; ++p) s += bf2f(dy[p * K + k]);
-    part[blockIdx.x * slice + k] = s;
-  }
 }
 
 // ------------------------------------------------------------ elementwise
@@ -1740,8 +1750,6 @@ int sps_nn_conv3x3_wgrad_bias(const void* x, const void* dpre, int n, int h,
   if (dbias) sp.count += cout;
   SPS_TRY(check_ws("sps_nn_conv3x3_wgrad", sp, workspace, ws_floats));
   int px;
-  // 16-byte loads in either kernel; the general one takes any alignment that
-  // its own loads do
   const int wc = wgrad_cols(h, w, cin, cout, &px);
   const int nchunks = (int)(npix / px);
   const int per = sp.per;
@@ -1761,10 +1769,12 @@ int sps_nn_conv3x3_wgrad_bias(const void* x, const void* dpre, int n, int h,
     else if (wc == 8) SPS_WGRAD_TILE(KT_, CT_, 8);                            \
     else if (w % 32 == 0)                                                     \
       conv_wgrad<KT_, CT_, true><<<grid, 256, 0, s>>>(                        \
-          xx, dd, n, h, w, cin, cout, workspace, sp.count, nchunks, per);     \
+          xx, dd, n, h, w, cin, cout, workspace, sp.count, nchunks, per,      \
+          dbias != nullptr);                                                  \
     else                                                                      \
       conv_wgrad<KT_, CT_, false><<<grid, 256, 0, s>>>(                       \
-          xx, dd, n, h, w, cin, cout, workspace, sp.count, nchunks, per);     \
+          xx, dd, n, h, w, cin, cout, workspace, sp.count, nchunks, per,      \
+          dbias != nullptr);                                                  \
   } while (0)
   if (kt == 64 && ct == 64)
     SPS_WGRAD(64, 64);
@@ -1777,11 +1787,6 @@ int sps_nn_conv3x3_wgrad_bias(const void* x, const void* dpre, int n, int h,
 #undef SPS_WGRAD
 #undef SPS_WGRAD_TILE
   SPS_TRY(launch_ok("sps_nn_conv3x3_wgrad"));
-  if (dbias && !wc) {
-    bias_partials<<<(unsigned)sp.blocks, 256, 0, s>>>(
-        dd, npix, cout, (int64_t)per * px, workspace + nw, sp.count);
-    SPS_TRY(launch_ok("sps_nn_conv3x3_wgrad_bias"));
-  }
   return add_parts(workspace, sp, dweight, s, nw, dbias);
 }
 

@@ -39,6 +39,28 @@ def test_weight_and_bias_gradients(gpu_lib, N, H, W, C, K):
     assert float((db.double() - dd.sum(0)).abs().max()) <= tol * scale
 
 
+@pytest.mark.parametrize("N,H,W,C,K", [(56, 24, 24, 256, 256), (8, 64, 64, 64, 64)])
+def test_the_bias_gradient_costs_no_pass_of_its_own(gpu_lib, N, H, W, C, K):
+    # general and tiled kernel: a product with ones beside nine of each tap's
+    # (1/9 of the products at most), against twice the time with a serial pass
+    x = torch.zeros(N, H, W, C, device="cuda", dtype=torch.bfloat16)
+    d = torch.zeros(N, H, W, K, device="cuda", dtype=torch.bfloat16)
+
+    def best(f):
+        times = []
+        for _ in range(8):
+            a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(20):
+                f(x, d, K)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    assert best(nn.conv3x3_wgrad_bias_raw) <= 1.5 * best(nn.conv3x3_wgrad_raw)
+
+
 # one run of 64 pixels, a part of one, rows shorter than a run, several and
 # more than 1024 workgroups' least; channels that leave waves idle
 @pytest.mark.parametrize("N,H,W,C", [(1, 8, 8, 32), (1, 5, 7, 8), (3, 3, 3, 16), (2, 9, 70, 24),
