@@ -46,9 +46,9 @@ int sps_nn_conv3x3(const void* x, int n, int h, int w, int cin,
 
 /* Weight gradients are deterministic: each workgroup reduces its share of
  * the pixels in a fixed order into its own partial gradient in a caller-owned
- * FP32 workspace; a fixed tree then adds the partials to dweight (16 or 4
- * equal ranges of them, each summed in order, then the ranges in order).  The
- * same inputs give the same bits on every call.  The workspace is scratch.
+ * FP32 workspace; a fixed tree then adds the partials to dweight, in FP64
+ * (16 or 4 equal ranges of them, each summed in order, then the ranges in
+ * order).  The same inputs give the same bits on every call.  The workspace is scratch.
  * sps_nn_wgrad_workspace gives the workspace size in floats for a layer
  * (kind SPS_NN_WGRAD_CONV with cin and cout, SPS_NN_WGRAD_IN1 with cout,
  * SPS_NN_WGRAD_OUT1 with cin); 0 for invalid sizes. */

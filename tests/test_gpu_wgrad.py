@@ -39,6 +39,29 @@ def test_weight_and_bias_gradients(gpu_lib, N, H, W, C, K):
     assert float((db.double() - dd.sum(0)).abs().max()) <= tol * scale
 
 
+# tiled, general and thin kernels, with 256 to 2048 partial sums
+@pytest.mark.parametrize("N,H,W,thin", [(32, 256, 256, False), (8, 100, 100, False),
+                                        (32, 256, 256, True), (8, 100, 90, True)])
+def test_bias_gradient_sums_keep_their_precision(gpu_lib, N, H, W, thin):
+    # positive sums of up to 2 million values: a workgroup's own sum is off by a
+    # few units of its last place, independent of the others', and their sum
+    # adds its one rounding, at most 2^-24 of every value
+    g = torch.Generator(device="cuda").manual_seed(H)
+    d = (torch.randn(N, H, W, 32, device="cuda", generator=g) * 0.1 + 0.05).to(torch.bfloat16)
+    if thin:
+        out = torch.zeros(10, 32, device="cuda")
+        s = torch.randn(N, H, W, device="cuda", generator=g)
+        ws = nn.wgrad_workspace(nn.WGRAD_IN1, N, H, W, 1, 32, "cuda")
+        nn._check(abi.load().sps_nn_conv3x3_in1_wgrad_bias(
+            nn._ptr(s), nn._ptr(d), N, H, W, 32, nn._ptr(out), nn._ptr(out[9]), nn._ptr(ws),
+            ws.numel(), nn._stream()))
+        db = out[9]
+    else:
+        db = nn.conv3x3_wgrad_bias_raw(torch.zeros_like(d), d, 32)[1]
+    want = d.double().sum((0, 1, 2))
+    assert float((db.double() - want).norm() / want.norm()) <= 2.0 ** -24
+
+
 @pytest.mark.parametrize("N,H,W,C,K", [(56, 24, 24, 256, 256), (8, 64, 64, 64, 64)])
 def test_the_bias_gradient_costs_no_pass_of_its_own(gpu_lib, N, H, W, C, K):
     # general and tiled kernel: a product with ones beside nine of each tap's
