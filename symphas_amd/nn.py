@@ -76,11 +76,20 @@ def conv3x3_wgrad_raw(x, dpre, K):
     return dw
 
 
+def _zero_gradients(wshape, K, device):
+    """Cleared FP32 gradients of a layer's weights and biases, each with a storage
+    and a version counter of its own (a parameter's .grad may be either), in one
+    launch."""
+    dw = torch.empty(wshape, device=device, dtype=torch.float32)
+    db = torch.empty(K, device=device, dtype=torch.float32)
+    torch._foreach_zero_((dw, db))
+    return dw, db
+
+
 def conv3x3_wgrad_bias_raw(x, dpre, K):
     """The weight gradient and the bias gradient from one read of dpre."""
     N, H, W, C = x.shape
-    g = torch.zeros(9 * K * C + K, device=x.device, dtype=torch.float32)
-    dw, db = g[:9 * K * C].view(9, K, C), g[9 * K * C:]
+    dw, db = _zero_gradients((9, K, C), K, x.device)
     ws = wgrad_workspace(WGRAD_CONV, N, H, W, C, K, x.device)
     _check(_lib().sps_nn_conv3x3_wgrad_bias(_ptr(x), _ptr(dpre), N, H, W, C, K, _ptr(dw), _ptr(db),
                                             _ptr(ws), ws.numel(), _stream()))
@@ -164,8 +173,7 @@ class _In1(torch.autograd.Function):
         dpre = silu_bwd_raw(dy, pre) if ctx.act == ACT_SILU else dy
         N, H, W = x.shape
         K = w.shape[1]
-        g = torch.zeros((10, K), device=x.device, dtype=torch.float32)
-        dw, db = g[:9], g[9]
+        dw, db = _zero_gradients((9, K), K, x.device)
         ws = wgrad_workspace(WGRAD_IN1, N, H, W, 1, K, x.device)
         _check(_lib().sps_nn_conv3x3_in1_wgrad_bias(_ptr(x.contiguous()), _ptr(dpre), N, H, W, K,
                                                     _ptr(dw), _ptr(db), _ptr(ws), ws.numel(),

@@ -115,3 +115,17 @@ def test_thin_gradients(gpu_lib, N, H, W, C):
             want = (v[..., None] * a.double()).sum((0, 1, 2))
             # sums of N*H*W unit products
             assert float((out[t].double() - want).abs().max()) <= tol * np.sqrt(N * H * W), (kind, t)
+
+
+def test_gradients_have_their_own_storage(gpu_lib):
+    # a parameter's .grad may be the tensor itself: no two share memory or a
+    # version counter
+    net = nn.UNet(seed=3).to("cuda")
+    x = torch.randn(2, 64, 64, device="cuda")
+    net(x).square().sum().backward()
+    grads = [p.grad for p in net.parameters()]
+    assert len({g.untyped_storage().data_ptr() for g in grads}) == len(grads)
+    assert all(g.untyped_storage().nbytes() == 4 * g.numel() for g in grads)
+    before = [g._version for g in grads]
+    grads[0].add_(1.0)
+    assert [g._version for g in grads[1:]] == before[1:]
