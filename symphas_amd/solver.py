@@ -130,7 +130,7 @@ class FDPlan:
             o_arr = np.ascontiguousarray(origin, dtype=np.float64)
             o = o_arr.ctypes.data_as(c_void_p)
         return _file_bytes(lambda buf, cap, n: self.lib.sps_fd_checkpoint_text(
-            self._h, int(index), o, buf, cap, n))
+            self._h, int(index), o, buf, cap, n), _checkpoint_cap(self.desc))
 
     def read_checkpoint(self, text: bytes) -> int:
         """Load a GNU checkpoint file into the field; returns its index."""
@@ -146,7 +146,7 @@ class FDPlan:
             o_arr = np.ascontiguousarray(origin, dtype=np.float64)
             o = o_arr.ctypes.data_as(c_void_p)
         return _file_bytes(lambda buf, cap, n: self.lib.sps_fd_plot_text(
-            self._h, int(fmt), o, buf, cap, n))
+            self._h, int(fmt), o, buf, cap, n), _plot_cap(self.desc))
 
     def checkpoint_xdr(self, index: int = 0, origin=None) -> bytes:
         """The field as the reference's XDR file (big-endian doubles)."""
@@ -205,42 +205,73 @@ def _origin_arg(origin):
     return arr, arr.ctypes.data_as(c_void_p)
 
 
+def _text_cap(desc, per_value: int, per_row: int, per_slice_header: int = 0) -> int:
+    n = [int(desc.n[a]) for a in range(desc.dim)]
+    sites = int(np.prod(n))
+    rows = sites // n[0]
+    slices = n[2] if desc.dim == 3 else 1
+    return per_value * sites + per_row * rows + slices * per_slice_header + 4096
+
+
+def _checkpoint_cap(desc) -> int:
+    """Bound of a checkpoint's length: 19 bytes per value ("-d.ddddddddddE+ddd "),
+    one newline per row, the header line."""
+    return _text_cap(desc, 19, 1)
+
+
+def _plot_cap(desc) -> int:
+    """Bound of a plot file's length, positions of up to 14 characters: 15 bytes
+    per value ("-d.ddddddE+ddd "), 15 per row (position column and newline), a
+    header line of 14 bytes per x position per z slice, blank lines."""
+    return _text_cap(desc, 15, 15, 14 * (int(desc.n[0]) + 1) + 2)
+
+
 _MADV_HUGEPAGE = 14
+_py = ctypes.pythonapi
+_bytes_new = ctypes.PYFUNCTYPE(c_void_p, c_void_p, ctypes.c_ssize_t)(
+    ("PyBytes_FromStringAndSize", _py))
+_bytes_address = ctypes.PYFUNCTYPE(c_void_p, c_void_p)(("PyBytes_AsString", _py))
+_bytes_resize = ctypes.PYFUNCTYPE(c_int, ctypes.POINTER(c_void_p), ctypes.c_ssize_t)(
+    ("_PyBytes_Resize", _py))
+_decref = ctypes.PYFUNCTYPE(None, c_void_p)(("Py_DecRef", _py))
 
 
-def _file_bytes(call) -> bytes:
+def _file_bytes(call, cap: int = 0) -> bytes:
     """The bytes of a file: call(buffer, capacity, length) as the C entry points
-    take them, asked for the length first and then to fill a bytes object of
-    that length in place (filling a larger array and copying it out touches
-    fresh memory twice).  Where the field was advanced between the two calls
-    the second text has a length of its own: a shorter one is cut to it, for a
-    longer one the call is made again.  Large objects ask for huge pages first,
-    as numpy's arrays do: the copy from the device into 4 KiB pages that do not
-    exist yet spends most of its time on their faults (73 MB: 17.5 ms, huge
-    pages 7.5).  Checkpoint text of 2048^2 FP32 values, in all: 26 ms that way,
-    8.7 this way."""
-    n = c_size_t(0)
-    abi.check(call(None, 0, byref(n)))
-    api = ctypes.pythonapi
-    new = ctypes.PYFUNCTYPE(ctypes.py_object, c_void_p, ctypes.c_ssize_t)(
-        ("PyBytes_FromStringAndSize", api))
-    address = ctypes.PYFUNCTYPE(c_void_p, ctypes.py_object)(("PyBytes_AsString", api))
+    take them fills a bytes object of cap bytes in place, which is then cut to
+    the file's length (filling an array and copying it out touches fresh memory
+    twice, and asking for the length first formats every value twice: GNU plot
+    text of 40x50x30 0.96 ms that way, 0.54 this way).  Where cap is 0, or turns
+    out too small, the entry point is asked for the length.  Large objects ask
+    for huge pages first, as numpy's arrays do: the copy from the device into
+    4 KiB pages that do not exist yet spends most of its time on their faults
+    (73 MB: 17.5 ms, huge pages 7.5)."""
+    n = c_size_t(cap)
+    if not cap:
+        abi.check(call(None, 0, byref(n)))
     while True:
         size = n.value
-        out = new(None, size)
-        at = address(out)
-        if size >= 1 << 22 and sys.platform == "linux":
-            page = mmap.PAGESIZE
-            first, end = -(-at // page) * page, (at + size) // page * page
-            madvise = ctypes.CDLL(None).madvise  # advice only: its result does not matter
-            madvise.argtypes = [c_void_p, c_size_t, c_int]
-            madvise(first, end - first, _MADV_HUGEPAGE)
-        rc = call(c_void_p(at), size, byref(n))
-        if rc == abi.OK and n.value <= size:
-            return out if n.value == size else out[:n.value]
+        obj = c_void_p(_bytes_new(None, size))
+        try:
+            at = _bytes_address(obj)
+            if size >= 1 << 22 and sys.platform == "linux":
+                page = mmap.PAGESIZE
+                first, end = -(-at // page) * page, (at + size) // page * page
+                madvise = ctypes.CDLL(None).madvise  # advice only: its result does not matter
+                madvise.argtypes = [c_void_p, c_size_t, c_int]
+                madvise(first, end - first, _MADV_HUGEPAGE)
+            rc = call(c_void_p(at), size, byref(n))
+            if rc == abi.OK:
+                if n.value != size:
+                    _bytes_resize(byref(obj), n.value)
+                return ctypes.cast(obj, ctypes.py_object).value
+        finally:
+            if obj:
+                _decref(obj)
+        error = abi.SpsError(rc, abi.load().sps_fd_last_error().decode())
         abi.check(call(None, 0, byref(n)))
         if n.value <= size:  # not for want of room
-            abi.check(rc)
+            raise error
 
 
 def checkpoint_progress(directory: str):
@@ -389,7 +420,7 @@ class MultiPlan:
         """Field `field` as the reference's GNU checkpoint file (device-formatted)."""
         keep, o = _origin_arg(origin)
         return _file_bytes(lambda buf, cap, n: self.lib.sps_fdm_checkpoint_text(
-            self._h, int(field), int(index), o, buf, cap, n))
+            self._h, int(field), int(index), o, buf, cap, n), _checkpoint_cap(self.desc))
 
     def read_checkpoint(self, field: int, text: bytes) -> int:
         idx = c_int(0)
@@ -400,7 +431,7 @@ class MultiPlan:
     def plot_text(self, field: int, fmt: int = abi.PLOT_GNU, origin=None) -> bytes:
         keep, o = _origin_arg(origin)
         return _file_bytes(lambda buf, cap, n: self.lib.sps_fdm_plot_text(
-            self._h, int(field), int(fmt), o, buf, cap, n))
+            self._h, int(field), int(fmt), o, buf, cap, n), _plot_cap(self.desc))
 
     def checkpoint_xdr(self, field: int, index: int = 0, origin=None) -> bytes:
         keep, o = _origin_arg(origin)
