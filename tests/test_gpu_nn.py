@@ -106,7 +106,8 @@ def test_thin_layers(gpu_lib, N, H, W, K):
     dpre = co.bf16_round(rnd((N, H, W, K), 15))
     dw = torch.zeros((9, K), device=DEV)
     ws = nn.wgrad_workspace(nn.WGRAD_IN1, N, H, W, 1, K, DEV)
-    nn._check(lib.sps_nn_conv3x3_in1_wgrad(nn._ptr(xt), nn._ptr(bf(dpre)), N, H, W, K,
+    dt = bf(dpre)  # held: the call gets the address only
+    nn._check(lib.sps_nn_conv3x3_in1_wgrad(nn._ptr(xt), nn._ptr(dt), N, H, W, K,
                                            nn._ptr(dw), nn._ptr(ws), ws.numel(), nn._stream()))
     refw = co.conv3x3_bwd_weight(x[..., None].astype(np.float64), dpre)[:, :, 0]
     assert np.allclose(dw.cpu().numpy(), refw, rtol=1e-4, atol=1e-4)
@@ -116,15 +117,17 @@ def test_thin_layers(gpu_lib, N, H, W, K):
     bo = np.array([0.3], np.float32)
     out = torch.empty((N, H, W), device=DEV)
     wot, bot = torch.from_numpy(wo).to(DEV), torch.from_numpy(bo).to(DEV)
-    nn._check(lib.sps_nn_conv3x3_out1(nn._ptr(bf(h)), N, H, W, K, nn._ptr(wot), nn._ptr(bot),
+    ht = bf(h)
+    nn._check(lib.sps_nn_conv3x3_out1(nn._ptr(ht), N, H, W, K, nn._ptr(wot), nn._ptr(bot),
                                       nn._ptr(out), nn._stream()))
     refo = co.conv3x3(h, wo[:, None, :].astype(np.float64), bo.astype(np.float64))[..., 0]
     assert np.allclose(out.cpu().numpy(), refo, rtol=1e-5, atol=1e-4)
     dy = rnd((N, H, W), 18).astype(np.float32)
+    dyt = torch.from_numpy(dy).to(DEV)
     dx = torch.empty((N, H, W, K), device=DEV, dtype=torch.bfloat16)
     dwo = torch.zeros((9, K), device=DEV)
     wso = nn.wgrad_workspace(nn.WGRAD_OUT1, N, H, W, K, 1, DEV)
-    nn._check(lib.sps_nn_conv3x3_out1_bwd(nn._ptr(bf(h)), nn._ptr(torch.from_numpy(dy).to(DEV)),
+    nn._check(lib.sps_nn_conv3x3_out1_bwd(nn._ptr(ht), nn._ptr(dyt),
                                           N, H, W, K, nn._ptr(wot), nn._ptr(dx), nn._ptr(dwo),
                                           nn._ptr(wso), wso.numel(), nn._stream()))
     refdx = co.conv3x3_bwd_data(dy[..., None].astype(np.float64), wo[:, None, :].astype(np.float64))
