@@ -21,9 +21,7 @@ template <typename T>
 bool launch_ref_set3d(int set, const T* in, T* out, const RefParams<T>& p,
                       const int (&kind)[3], hipStream_t s) {
   if ((p.L != 7 && p.L != 15) || ((set & kSBilap) && p.B != 25)) return false;
-  // a field this small gives the stream too few waves to cover the latency of
-  // a plane (32^3 FP32 Model B: 7.8 us per step, the one-site kernel 7.0)
-  if ((int64_t)p.n[0] * p.n[1] * p.n[2] < 40000) return false;
+  if (one_site_step3d(p.n[0], p.n[1], p.n[2], sizeof(T))) return false;
   switch (set) {
 #define SPS_SET3(SET)                                        \
   case SET:                                                  \

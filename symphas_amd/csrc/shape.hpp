@@ -1,4 +1,4 @@
-// shape.hpp - launch shapes of the fused streams before any tuning.
+// shape.hpp - launch shapes of the streams before any tuning.  Host code only.
 //
 // A launch of a stream is one wave per (strip, chunk).  Every wave walks the
 // rows (2D) or planes (3D) of its chunk plus the pipeline's fill, and a SIMD
@@ -94,6 +94,17 @@ inline StreamShape stream_shape3d(int X, int Y, int Z, int R, int esize,
     }
   }
   return best;
+}
+
+// Whether a 3D reference-order step runs one thread per site: while all its
+// workgroups of 64 x 4 sites are resident at once (two per CU in FP32, one in
+// FP64), the launch is one chain of loads and sums, where the plane stream walks
+// at least six planes.  <15,10,25> Model B, us per step, one site / stream: FP32
+// 44^3 (484 workgroups) 7.2 / 7.6, 48^3 (576) 11.5 / 7.6; FP64 36^3 (324) 13.8 /
+// 8.3, and 7.9 at 32^3 (256).
+inline bool one_site_step3d(int X, int Y, int Z, int esize) {
+  const int64_t workgroups = (int64_t)((X + 63) / 64) * ((Y + 3) / 4) * Z;
+  return workgroups <= (esize == 4 ? 512 : 256);
 }
 
 }  // namespace sps

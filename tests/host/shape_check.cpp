@@ -1,0 +1,18 @@
+// Prints what the launch-shape rules of shape.hpp pick, one line per line of
+// standard input (a rule's name and its arguments).
+#include <cstdio>
+#include <cstring>
+
+#include "../../symphas_amd/csrc/shape.hpp"
+
+int main() {
+  char rule[32];
+  int X, Y, Z, esize;
+  while (std::scanf("%31s", rule) == 1) {
+    if (!std::strcmp(rule, "one_site") && std::scanf("%d%d%d%d", &X, &Y, &Z, &esize) == 4)
+      std::printf("%d\n", sps::one_site_step3d(X, Y, Z, esize) ? 1 : 0);
+    else
+      return 1;
+  }
+  return 0;
+}

@@ -58,7 +58,9 @@ def test_step_equals_one_site_kernel(gpu_lib, shape, dtype):
 
 
 @pytest.mark.parametrize("dtype", [abi.F32, abi.F64])
-@pytest.mark.parametrize("shape", [(3, 4, 5), (3, 4, 3500), (60, 5, 150), (61, 220, 3), (125, 33, 26)])
+# up to 512 workgroups (FP32; FP64 256) the one-site kernel takes the step
+@pytest.mark.parametrize("shape", [(3, 4, 5), (3, 4, 3500), (60, 5, 150), (61, 220, 3), (125, 33, 26),
+                                   (60, 5, 257), (61, 685, 3), (125, 33, 29)])
 def test_3d_step_equals_one_site_kernel(gpu_lib, shape, dtype):
     print("[case] ref stream 3D", shape, dtype, flush=True)
     t = np.float32 if dtype == abi.F32 else np.float64
