@@ -66,53 +66,34 @@ struct sps_fd_plan {
   void drop_graphs();
 
   // Launch shape before any tuning (shape.hpp).  2D: four steps per launch,
-  // the best at every size measured.  3D: t of the (steps, rows) shapes as
-  // fitted over 32^3 .. 256^3 and uneven boxes (FP32 12 rows at two steps fill
-  // two waves per SIMD; FP64 rings of two steps hold four rows).
+  // the best at every size measured.  3D at radius one: t of the (steps, rows)
+  // shapes as fitted over 32^3 .. 256^3 and uneven boxes.
   void choose_default_shape() {
-    const int R = fc64.radius;
+    const int R = fc64.radius, X = d.n[0], Y = d.n[1], Z = d.n[2];
     sps::StreamShape s;
     if (d.dim == 2) {
-      s = sps::stream_shape2d(d.n[0], d.n[1], 4, R, (int)esize);
+      s = sps::stream_shape2d(X, Y, 4, R, (int)esize);
+    } else if (R == 2) {
+      s = sps::radius_two_shape3d(X, Y, Z, (int)esize);
     } else if (d.dtype == SPS_F32) {
-      static const sps::Stream3DCand c[2][4] = {
-          {{2, 4, 0.258}, {2, 6, 0.333}, {2, 8, 0.433}, {2, 12, 0.603}},
-          {{2, 4, 0.422}, {2, 6, 0.513}, {2, 8, 0.652}, {2, 12, 0.836}}};
-      // The halo rows of low waves are read again from the last-level cache or
-      // HBM once both fields outgrow the L2s by far: 256^3 at radius two, 6
-      // rows 25.5 us per step, 12 rows 24.0; 300x280x260, 8 rows 29.2, 12 rows 27.6.
-      const double both = 8.0 * (double)nsites;
-      const int skip = R == 1 ? 0 : both > 160e6 ? 3 : both > 100e6 ? 2 : 0;
-      s = sps::stream_shape3d(d.n[0], d.n[1], d.n[2], R, 4, 1, c[R - 1] + skip, 4 - skip,
-                              1.4);
-    } else if (R == 1) {
+      static const sps::Stream3DCand c[4] = {
+          {2, 4, 0.258}, {2, 6, 0.333}, {2, 8, 0.433}, {2, 12, 0.603}};
+      s = sps::stream_shape3d(X, Y, Z, R, 4, 1, c, 4, 1.4);
+    } else {
       // Two steps of 4 rows always: one step of 8 rows was 18.6 us per step on
       // 61x500x200, two of 4 rows 15.9.  Even splits of Z, the tallest of equal
       // cost (fewer planes read twice where HBM is the bound).
       static const sps::Stream3DCand two = {2, 4, 0.418};
       double least = 0;
-      for (int m = 1; m <= d.n[2]; ++m) {
-        const int tz = (d.n[2] + m - 1) / m;
+      for (int m = 1; m <= Z; ++m) {
+        const int tz = (Z + m - 1) / m;
         if (tz > 1024) continue;
-        const double cost = sps::stream_cost3d(d.n[0], d.n[1], d.n[2], R, 8, 1, two, tz, 1.1);
+        const double cost = sps::stream_cost3d(X, Y, Z, R, 8, 1, two, tz, 1.1);
         if (least == 0 || cost < least * 0.999) {
           least = cost;
           s = sps::StreamShape{2, 4, tz, 1};
         }
       }
-    } else {
-      // The radius-two rings of two FP64 steps leave room for one wave per
-      // SIMD: a second one runs after it, not beside it (q = 1).  256^3:
-      // 86-plane chunks 43.9 us per step, 43-plane chunks (two waves) 49.7.
-      static const sps::Stream3DCand two = {2, 4, 0.92};
-      static const sps::Stream3DCand one[3] = {{1, 4, 0.47}, {1, 8, 0.79}, {1, 12, 1.10}};
-      const int X = d.n[0], Y = d.n[1], Z = d.n[2];
-      s = sps::stream_shape3d(X, Y, Z, R, 8, 1, &two, 1, 1.0);
-      const sps::StreamShape o = sps::stream_shape3d(X, Y, Z, R, 8, 1, one, 3, 1.1);
-      const sps::Stream3DCand& oc = one[o.rows == 4 ? 0 : o.rows == 8 ? 1 : 2];
-      if (sps::stream_cost3d(X, Y, Z, R, 8, 1, oc, o.planes, 1.1) <
-          sps::stream_cost3d(X, Y, Z, R, 8, 1, two, s.planes, 1.0))
-        s = o;
     }
     K = s.steps;
     TY = s.rows;
