@@ -13,17 +13,15 @@
 // replayed.
 #include <algorithm>
 #include <cstring>
-#include <functional>
-#include <map>
 #include <new>
 #include <vector>
 
+#include "batch_items.hpp"
 #include "common.hpp"
 #include "energy.hpp"
 #include "fused_tile.hpp"
 #include "plan.hpp"
 #include "reduce_rows.hpp"
-#include "shape.hpp"
 
 namespace sps {
 namespace {
@@ -35,21 +33,6 @@ struct BatchInst {
   double h, divh;
   FusedCoef<float> c;
 };
-
-struct BatchItem {
-  int inst, y0, ty, strip;
-};
-
-// Strip geometry of the 2-values-per-lane stream (fused_tile.hpp): a wave
-// covers (64 - 2*HL)*2 columns and HL halo lanes per side carry the K*R
-// columns the K fused steps reach.
-constexpr int kBatchVec = 2;
-__host__ __device__ constexpr int batch_halo_lanes(int K, int R) {
-  return (K * R + kBatchVec - 1) / kBatchVec;
-}
-__host__ __device__ constexpr int batch_strip_width(int K, int R) {
-  return (64 - 2 * batch_halo_lanes(K, R)) * kBatchVec;
-}
 
 template <int K, int R, bool HASA>
 __device__ __forceinline__ void run_strip(const BatchInst& I, int parity,
@@ -191,109 +174,32 @@ struct sps_fd_batch {
   int radius_of(int i) const {
     return (h_insts[i].kind == 1 || h_insts[i].kind == 2) ? 2 : 1;
   }
-  // cost of streaming a chunk of ty rows, K steps: the rows and the fill, a
-  // radius-two row 10 to a radius-one row's 9
-  static int item_cost(int k, int R, int ty) {
-    return (ty + 2 * k * R) * (R == 2 ? 10 : 9);
-  }
+  // Item height before any tuning.  256 mixed instances, us per 4-step launch at
+  // 48 / 64 / 86 / 96 / 128 rows: 45.8 / 47.3 / 45.2 / 45.5 / 49.2 (96 is
+  // picked); 75 of them at 43 / 47 / 64: 20.6 / 19.2 / 22.5 (47); 170 at 64 / 96
+  // / 103: 32.2 / 36.6 / 33.5 (103).
+  void choose_rows() { TY = batch_rows(sides(), K); }
 
-  // Item height before any tuning: between the mean load of a SIMD and the
-  // load of one that gets the first item of every layer of kSimds items, taken
-  // costliest first; a lone item's rows cost 1.5 of a shared one's (their
-  // latency shows).  256 mixed instances, us per 4-step launch at 48 / 64 / 86
-  // / 96 / 128 rows: 48.2 / 48.8 / 45.3 / 46.3 / 49.6 (96 is picked); the list
-  // sorted over the whole chip instead of per XCD 53.9 / 53.1 / 49.3 / 52.1 /
-  // 51.4.
-  void choose_rows() {
-    int64_t least = 0;
-    for (int rows : {4, 6, 8, 12, 16, 24, 32, 43, 48, 64, 86, 96, 103, 128, 171, 256, 512}) {
-      std::map<int, int64_t, std::greater<int>> hist;  // cost -> items
-      for (int i = 0; i < count; ++i) {
-        const int R = radius_of(i), W = batch_strip_width(K, R);
-        const int X = descs[i].n[0], Y = descs[i].n[1];
-        const int64_t strips = (X + W - 1) / W;
-        if (Y / rows) hist[item_cost(K, R, rows)] += strips * (Y / rows);
-        if (Y % rows) hist[item_cost(K, R, Y % rows)] += strips;
-      }
-      int64_t layers = 0, all = 0, next = 0, seen = 0;
-      for (const auto& h : hist) {
-        seen += h.second;
-        all += h.first * h.second;
-        for (; next < seen; next += kSimds) layers += h.first;
-      }
-      const int64_t cost = std::max((all / kSimds + layers) / 2,
-                                    hist.begin()->first * (int64_t)3 / 2);
-      if (least == 0 || cost < least) {
-        least = cost;
-        TY = rows;
-      }
-    }
+  std::vector<BatchSides> sides() const {
+    std::vector<BatchSides> v;
+    for (int i = 0; i < count; ++i)
+      v.push_back(BatchSides{descs[i].n[0], descs[i].n[1], radius_of(i)});
+    return v;
   }
 
   // The item list of each steps-per-launch, for the batch's item height.
   int build_items() {
-    constexpr int kXcds = 8, kWaves = 4;  // kWaves: of a workgroup
+    constexpr int kWaves = 4;  // of a workgroup
+    const std::vector<BatchSides> inst = sides();
     for (int k = 1; k <= 4; ++k) {
-      // units of work that stay together: an instance, or a piece of one that
-      // is more than 1/64 of the batch
-      struct Unit {
-        int64_t cost;
-        std::vector<BatchItem> items;
-      };
-      auto cost = [&](const BatchItem& it) {
-        return (int64_t)item_cost(k, radius_of(it.inst), it.ty);
-      };
-      std::vector<Unit> units;
-      int64_t total = 0;
-      for (int i = 0; i < count; ++i) {
-        const int W = batch_strip_width(k, radius_of(i));
-        const int X = descs[i].n[0], Y = descs[i].n[1];
-        units.push_back(Unit{0, {}});
-        for (int st = 0; st * W < X; ++st)
-          for (int y0 = 0; y0 < Y; y0 += TY) {
-            const BatchItem it{i, y0, std::min(TY, Y - y0), st};
-            units.back().items.push_back(it);
-            units.back().cost += cost(it);
-          }
-        total += units.back().cost;
-      }
-      std::vector<Unit> pieces;
-      for (Unit& u : units) {
-        if (u.cost * 64 <= total) {
-          pieces.push_back(std::move(u));
-          continue;
-        }
-        pieces.push_back(Unit{0, {}});
-        for (const BatchItem& it : u.items) {
-          if (pieces.back().cost * 64 > total) pieces.push_back(Unit{0, {}});
-          pieces.back().items.push_back(it);
-          pieces.back().cost += cost(it);
-        }
-      }
-      // the largest first, each to the XCD with the least so far
-      std::stable_sort(pieces.begin(), pieces.end(),
-                       [](const Unit& a, const Unit& b) { return a.cost > b.cost; });
-      Unit xcd[kXcds];
-      for (Unit& x : xcd) x.cost = 0;
-      for (const Unit& u : pieces) {
-        Unit* least = std::min_element(
-            xcd, xcd + kXcds, [](const Unit& a, const Unit& b) { return a.cost < b.cost; });
-        least->cost += u.cost;
-        least->items.insert(least->items.end(), u.items.begin(), u.items.end());
-      }
+      const BatchLists xcd = batch_lists(inst, k, TY);
       size_t longest = 0;
-      for (Unit& x : xcd) {
-        std::stable_sort(x.items.begin(), x.items.end(),
-                         [&](const BatchItem& a, const BatchItem& b) {
-                           return cost(a) > cost(b);
-                         });
-        longest = std::max(longest, x.items.size());
-      }
+      for (const auto& x : xcd) longest = std::max(longest, x.size());
       std::vector<BatchItem> items;
       for (size_t q = 0; q < longest; q += kWaves)
-        for (const Unit& x : xcd)
+        for (const auto& x : xcd)
           for (size_t w = q; w < q + kWaves; ++w)
-            items.push_back(w < x.items.size() ? x.items[w] : BatchItem{0, 0, 0, 0});
+            items.push_back(w < x.size() ? x[w] : BatchItem{0, 0, 0, 0});
       if (d_items[k - 1]) (void)hipFree(d_items[k - 1]);
       d_items[k - 1] = nullptr;
       nitems[k - 1] = (int)items.size();

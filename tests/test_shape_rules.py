@@ -1,6 +1,7 @@
 """The launch-shape rules (symphas_amd/csrc/shape.hpp), compiled for the host,
 against times measured on an MI355X: what a rule picks is no slower than what it
 passes over."""
+import random
 import shutil
 import subprocess
 from pathlib import Path
@@ -114,3 +115,36 @@ def test_radius_two_is_no_slower_than_one_round(pick):
         assert picked == shape, (es, n)
         # 1%: two runs of one shape differ by as much
         assert times[0] <= 1.01 * one[0] and times[1] <= 1.01 * one[1], (es, n)
+
+
+# batches of equal instances: number, side, radius, us per launch of four steps
+# by item height
+BATCHES = [
+    (64, 256, 1, {8: 12.05, 10: 12.16, 13: 12.46, 16: 11.91, 24: 13.12, 26: 12.39, 32: 14.05,
+                  64: 15.44, 128: 25.78}),
+    (4, 1024, 2, {21: 15.58, 23: 16.26, 24: 16.69, 32: 18.45, 43: 16.29, 45: 15.66, 64: 18.78,
+                  128: 30.59}),
+    (1000, 128, 2, {24: 57.38, 32: 51.05, 64: 44.86, 86: 44.95, 96: 43.46, 128: 45.33}),
+    (1, 512, 2, {4: 5.43, 6: 5.90, 8: 6.24, 16: 8.47, 32: 11.22, 64: 16.69}),
+]
+
+
+def test_batch_heights_split_the_sides(pick):
+    got = pick([f"batch {n} " + f"{side} {side} {r} " * n for n, side, r, _ in BATCHES])
+    for (n, side, r, us), (rows,) in zip(BATCHES, got):
+        assert rows in {-(-side // m) for m in range(1, side)}, (n, side)
+        assert us[rows] <= 1.05 * min(us.values()), (n, side)
+    # sides of no listed height, and sides below the least height
+    (a,), (b,) = pick(["batch 3 100 300 2 220 220 1 150 100 2", "batch 2 8 3 2 6 3 1"])
+    assert any(a in {-(-y // m) for m in range(1, y)} for y in (300, 220, 100)) and b == 4
+
+
+def test_batch_cost_is_that_of_the_lists(pick):
+    # mixed sides, one instance that is split, two instances, one
+    rng = random.Random(3)
+    batches = [[(2 * rng.randrange(2, 260), rng.randrange(3, 520), rng.randrange(1, 3))
+                for _ in range(n)] for n in (120, 40, 2, 1)]
+    batches.append([(2048, 1500, 2)] + [(128, 128, 1)] * 30)
+    lines = [f"launch_cost {k} {rows} {len(b)} " + " ".join(f"{x} {y} {r}" for x, y, r in b)
+             for b in batches for k in (1, 2, 3, 4) for rows in (4, 17, 64, 103, 512)]
+    assert all(by_count == by_list for by_count, by_list in pick(lines))
