@@ -268,7 +268,10 @@ def _file_bytes(call, cap: int = 0) -> bytes:
         finally:
             if obj:
                 _decref(obj)
-        error = abi.SpsError(rc, abi.load().sps_fd_last_error().decode())
+        try:
+            abi.check(rc)
+        except abi.SpsError as exc:
+            error = exc
         abi.check(call(None, 0, byref(n)))
         if n.value <= size:  # not for want of room
             raise error
